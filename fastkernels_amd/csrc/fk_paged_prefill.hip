@@ -28,6 +28,12 @@ void launch_prefill_d(bool paged, bool fp8, bool split, const PrefillParams& P, 
     launch_prefill_bf16<D, D>(paged, split, P, grid, bt, cu_q, cu_k, stream);
 }
 
+// Query tokens per work-group.
+int64_t prefill_wg_tokens(int gqa, int head_size, int head_size_v) {
+  const int hw = gqa < kPrefillWaves ? gqa : kPrefillWaves;
+  return static_cast<int64_t>(kPrefillWaves / hw) * 16 * col_blocks_for(head_size, head_size_v);
+}
+
 // Launch shape of a prefill call, from the host-side bounds alone (the plan
 // entry point and the launch agree on it).
 struct PrefillShape {
@@ -44,8 +50,7 @@ PrefillShape prefill_shape(bool paged, bool fp8, int64_t batch, int64_t max_seql
   PrefillShape sh;
   const int gqa = num_heads / num_kv_heads;
   const int hw = gqa < kPrefillWaves ? gqa : kPrefillWaves;  // query heads per work-group
-  const int64_t wg_tokens =
-      static_cast<int64_t>(kPrefillWaves / hw) * 16 * col_blocks_for(head_size, head_size_v);
+  const int64_t wg_tokens = prefill_wg_tokens(gqa, head_size, head_size_v);
   sh.qblocks = (max_seqlen_q + wg_tokens - 1) / wg_tokens;
   sh.hsplit = (gqa + hw - 1) / hw;
   // Key split when the 4-wave launch would leave SIMDs with one wave: fewer
@@ -324,8 +329,17 @@ int prefill_entry(const char* name, bool paged, void* out, int64_t out_row_strid
   P.num_heads = num_heads;
   FK_REQUIRE(qblocks <= 65535, "%s: max_seqlen_q %lld needs more than 65535 query blocks", name,
              (long long)max_seqlen_q);
-  const dim3 grid(static_cast<unsigned>(num_kv_heads * sh.hsplit), static_cast<unsigned>(batch),
-                  static_cast<unsigned>(qblocks * sh.xs));
+  // Longest items first: up to 64 sequences (one per lane of the kernel's ordering).
+  // Items: at most ceil(q_len / block) per sequence.
+  const int64_t wg_tokens = prefill_wg_tokens(P.gqa, head_size, head_size_v);
+  int64_t items = batch * qblocks;
+  if (total_q > 0) items = std::min(items, total_q / wg_tokens + batch);
+  P.lpt = (batch <= 64 && items * sh.xs <= 65535) ? static_cast<int>(batch) : 0;
+  const dim3 grid =
+      P.lpt ? dim3(static_cast<unsigned>(num_kv_heads * sh.hsplit),
+                   static_cast<unsigned>(items * sh.xs), 1)
+            : dim3(static_cast<unsigned>(num_kv_heads * sh.hsplit), static_cast<unsigned>(batch),
+                   static_cast<unsigned>(qblocks * sh.xs));
   hipStream_t s = as_stream(stream);
   const bool split = sh.ks > 1;
   if (head_size == head_size_v && (head_size == 64 || head_size == 128 || head_size == 256)) {

@@ -96,6 +96,11 @@ struct PrefillParams {
   void* part;
   int64_t part_rows;  // rows of q (at least cu_seqlens_q[batch])
   int num_heads;
+  // Longest items first (0: off, the grid's y is the sequence and z the query
+  // block): the number of sequences, at most 64; the grid's y is then the rank of
+  // the item (sequence, query block or pair) in descending order of the
+  // sequence's key stages (x P.xs key parts, the part fastest).
+  int lpt;
 };
 
 // Floats of the partial state per (part, row, head) besides O.
@@ -402,6 +407,45 @@ __device__ __forceinline__ void lds_v_slice2(const uint8_t* buf, int tt, int d, 
   }
 }
 
+// Item `rank` (sequence b, its item x: a query block or pair of blocks) of the
+// launch, the sequences in descending order of the key stages one of their items
+// streams; false past the last item.  Work-groups are dispatched in grid order,
+// so the longest run first and the short ones fill the gaps at the end; the
+// items of one sequence stay adjacent, so that work-groups running at the same
+// time share its keys in L2.  Lane b holds sequence b (P.lpt of them, at most
+// 64): its start in the order is the item count of the sequences before it.
+__device__ __forceinline__ bool lpt_item(const PrefillParams& P, const int32_t* __restrict__ cu_q,
+                                         const int32_t* __restrict__ cu_k, int wg_tokens,
+                                         int rank, int& b, int& x) {
+  if (P.lpt == 1) {  // one sequence: its blocks in order (the caller checks the count)
+    b = 0;
+    x = rank;
+    return true;
+  }
+  const int lane = threadIdx.x & 63;
+  const int lb = min(lane, P.lpt - 1);
+  const int q_len = cu_q[lb + 1] - cu_q[lb];
+  const int k_len = cu_k[lb + 1] - cu_k[lb];
+  const int nqb = (q_len + wg_tokens - 1) / wg_tokens;
+  const bool paired = P.causal && k_len - q_len < q_len;
+  const int n = lane < P.lpt ? (paired ? (nqb + 1) / 2 : nqb) : 0;
+  int keys = min(max(k_len, 0), 1 << 28) + (paired ? wg_tokens : 0);
+  if (P.window_left >= 0)
+    keys = min(keys, (paired ? 2 : 1) * (min(P.window_left, INT_MAX / 8) + wg_tokens));
+  const int key = (keys / kStageKeys) * 64 + (63 - lane);  // distinct: ties keep their order
+  int start = 0;
+  for (int j = 0; j < P.lpt; ++j) {
+    const int nj = __builtin_amdgcn_readlane(n, j);
+    const int kj = __builtin_amdgcn_readlane(key, j);
+    start += kj > key ? nj : 0;
+  }
+  const uint64_t hit = __ballot(rank >= start && rank < start + n);
+  if (hit == 0) return false;
+  b = __builtin_ctzll(hit);
+  x = rank - __builtin_amdgcn_readlane(start, b);
+  return true;
+}
+
 // Work-group = kPrefillWaves waves over one kv head: hw query heads of its group
 // times qs = kPrefillWaves / hw blocks of kQTokens query tokens (a group larger
 // than kPrefillWaves heads spans hsplit work-groups).  All waves share the K/V
@@ -469,12 +513,23 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
   // parts, the part fastest).  The block index varies slowest, so the
   // work-groups that have work (low z when blocks are paired) are dispatched
   // first and spread over every CU.
-  const int b = blockIdx.y;
   const int hw = P.gqa < kPrefillWaves ? P.gqa : kPrefillWaves;  // heads per work-group
   const int qs = kPrefillWaves / hw;                             // query blocks per work-group
   const int hsplit = (P.gqa + hw - 1) / hw;
   const int h = blockIdx.x / hsplit;
   const int head0 = (blockIdx.x - h * hsplit) * hw;
+  const int wg_tokens = qs * kQT;
+  const int xs = P.xs;
+  int b = blockIdx.y;
+  int x, xpart;  // this work-group's item of the sequence and its key part
+  if (P.lpt) {
+    const int rank = static_cast<int>(blockIdx.y) / xs;
+    xpart = static_cast<int>(blockIdx.y) - rank * xs;
+    if (!lpt_item(P, cu_q, cu_k, wg_tokens, rank, b, x)) return;
+  } else {
+    x = static_cast<int>(blockIdx.z) / xs;
+    xpart = static_cast<int>(blockIdx.z) - x * xs;
+  }
   const int q_start = cu_q[b];
   const int q_len = cu_q[b + 1] - q_start;
   const int k_start = cu_k[b];
@@ -487,12 +542,8 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
   // long tail on its own; the upper half of the grid then has nothing to do.
   // Otherwise the blocks' key counts are close, and work-group x takes block
   // nqb - 1 - x alone (the heaviest first), keeping twice the work-groups.
-  const int wg_tokens = qs * kQT;
   const int nqb = (q_len + wg_tokens - 1) / wg_tokens;
   const bool paired = P.causal && k_len - q_len < q_len;
-  const int xs = P.xs;
-  const int x = static_cast<int>(blockIdx.z) / xs;
-  const int xpart = static_cast<int>(blockIdx.z) - x * xs;  // this work-group's key part
   if (x >= (paired ? (nqb + 1) / 2 : nqb)) return;  // uniform over the work-group
   const int wave_id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int half = kKS > 1 ? wave_id / kPrefillWaves : 0;  // key-split half
