@@ -179,11 +179,6 @@ constexpr int kPrefillWaves = 4;               // waves per work-group
 #define FK_PREFILL_ALT_ORDER 1
 #endif
 
-// fp8 pages: each stage converted once into bf16 LDS buffers (1), or every
-// wave dequantising the K / V bytes it reads (0).
-#ifndef FK_PREFILL_FP8_CONVERT
-#define FK_PREFILL_FP8_CONVERT 1
-#endif
 // Keys per LDS stage (a multiple of 32).  Measured on MI355X (bf16, 1x2048,
 // 4x512 over 4096, 16x512 prompts): 32 keys 102 / 220 / 89 us against 117 /
 // 244 / 99 us for 64; again with the current loop, 88 / 187 / 83 against
@@ -299,14 +294,6 @@ __device__ __forceinline__ void lds_dma16_s(const uint8_t* base, uint32_t off, u
       : "memory");
 }
 
-// Value of `x` held by lane 4g + i (g = this lane's row group, lanes 16g ..
-// 16g + 15), for the O row 4g + i this lane accumulates: one cross-lane read
-// (ds_bpermute) rather than four readlanes and a select chain, which the
-// compiler turns into branches.
-__device__ __forceinline__ float row_from(float x, int g, int i) {
-  return __int_as_float(__builtin_amdgcn_ds_bpermute((4 * g + i) * 4, __float_as_int(x)));
-}
-
 // LDS byte address of a pointer into a __shared__ array.
 __device__ __forceinline__ uint32_t lds_addr_of(const uint8_t* p) {
   return static_cast<uint32_t>(
@@ -321,25 +308,6 @@ constexpr int split_exchange_floats() {
   return kCB * (DVP / 16) * 64 * 4 + kCB * 64 * 4 + kCB * 64;
 }
 
-// Tile tt (rows 16 tt .. 16 tt + 15) of a staged buffer in the register layout
-// a global load of the tile would give (DTile, fk_attn_tile.h): the K rows (t.k)
-// and, for fp8 stages, the V rows (t.v), read separately so that a caller can
-// keep them apart in time.
-template <bool kFp8, int D>
-__device__ __forceinline__ void lds_tile_k(const uint8_t* buf, int tt, int r, int g,
-                                           DTile<kFp8, D>& t) {
-  using S = Stage<kFp8, D, D>;
-  const int kr = 16 * tt + r;
-  if constexpr (!kFp8) {
-#pragma unroll
-    for (int c = 0; c < D / 32; ++c)
-      t.k[c] = *reinterpret_cast<const uint4*>(buf + S::offset(0, kr, 4 * c + g));
-  } else {
-#pragma unroll
-    for (int c = 0; c < D / 64; ++c)
-      t.k[c] = *reinterpret_cast<const uint4*>(buf + S::offset(0, kr, (D / 64) * g + c));
-  }
-}
 // K operand chunks of tile tt of a bf16 stage: chunk c = dims 32c + 8g .. +7 of key
 // row 16 tt + r, for c < qk_extent(D) / 32; chunks past the row's data are zero.
 template <int D, int DV>
@@ -353,18 +321,6 @@ __device__ __forceinline__ void lds_k_chunks(const uint8_t* buf, int tt, int r, 
     // (c is known after unrolling: only the chunk that crosses the row's end selects.)
     kc[c] = (4 * c + 3 < S::kKReal || 4 * c + g < S::kKReal) ? v : make_uint4(0, 0, 0, 0);
   }
-}
-
-// fp8 V rows 4g + i: lane r's D / 16 bytes (dims (D/16) r ..), inside one chunk.
-template <bool kFp8, int D>
-__device__ __forceinline__ void lds_tile_v(const uint8_t* buf, int tt, int r, int g,
-                                           DTile<kFp8, D>& t) {
-  static_assert(kFp8, "bf16 V rows are read with lds_v_slice");
-  using S = Stage<kFp8, D, D>;
-  const int byte = (D / 16) * r;
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-    ld_words(buf + S::offset(1, 16 * tt + 4 * g + i, byte >> 4) + (byte & 15), t.v[i]);
 }
 
 // P.V operand of the 16-dim slice d of tile tt (bf16 stages), read with the LDS
@@ -414,6 +370,11 @@ __device__ __forceinline__ void lds_v_slice2(const uint8_t* buf, int tt, int d, 
 // items of one sequence stay adjacent, so that work-groups running at the same
 // time share its keys in L2.  Lane b holds sequence b (P.lpt of them, at most
 // 64): its start in the order is the item count of the sequences before it.
+// With the sequences side by side in the grid (block index slowest), the last
+// blocks dispatched were the longest sequences': same box, us, before -> after:
+// 5 ragged chunks (418 .. 700 over 3191 .. 6000) 384 -> 325, a vision encoder's
+// 1116 .. 3000 tokens (16 heads of 80) 307 -> 224, 13 fp8 prompts of 160 .. 1100
+// 152 -> 139, MLA chunks (2 x 16 heads 192 / 128) 292 -> 249, one prompt unchanged.
 __device__ __forceinline__ bool lpt_item(const PrefillParams& P, const int32_t* __restrict__ cu_q,
                                          const int32_t* __restrict__ cu_k, int wg_tokens,
                                          int rank, int& b, int& x) {
@@ -471,10 +432,9 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
   // with two work-groups per CU, so one bf16 buffer serves the stages in turn
   // (kConv1: converted after every wave is done with the stage before, a second
   // barrier per stage).
-  constexpr bool kConv = kFp8 && FK_PREFILL_FP8_CONVERT && D <= 128;
-  constexpr bool kConv1 = kFp8 && FK_PREFILL_FP8_CONVERT && D > 128;
-  constexpr bool kFp8T = kFp8 && !kConv && !kConv1;  // fp8 tiles in the compute path
-  using SB = Stage<kFp8T, D, DV>;         // the layout the compute path reads
+  constexpr bool kConv = kFp8 && D <= 128;
+  constexpr bool kConv1 = kFp8 && D > 128;
+  using SB = Stage<false, D, DV>;         // the layout the compute path reads
   static_assert(kKS == 1 || (kKS == 2 && (D <= 192 || kPaged)),
                 "key split: two halves, head size <= 192 (256 with paged keys)");
   constexpr int kCB = col_blocks_for(D, DV);  // 16-query column blocks per wave
@@ -635,6 +595,33 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
     }
   };
 
+  // Writes the query row a lane holds (column r of an O^T tile set: slice d's dims
+  // 16 d + 4 g .. + 3) as bf16, each value times f.  Slices go in pairs: swapping
+  // rows of 16 lanes between them leaves 8 adjacent dims per lane (even g: of the
+  // first slice, odd g: of the second), one 16-byte store per pair.
+  auto write_row = [&](uint16_t* row, const floatx4_t (&ov)[kVS], float f, bool ok)
+                       __attribute__((always_inline)) {
+    auto packed = [&](int d) {
+      const bf16x2_t a = {static_cast<__bf16>(ov[d][0] * f), static_cast<__bf16>(ov[d][1] * f)};
+      const bf16x2_t b = {static_cast<__bf16>(ov[d][2] * f), static_cast<__bf16>(ov[d][3] * f)};
+      return make_uint2(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b));
+    };
+#pragma unroll
+    for (int d = 0; d + 1 < kVS; d += 2) {
+      const uint2 a = packed(d), c = packed(d + 1);
+      const auto x = __builtin_amdgcn_permlane16_swap(a.x, c.x, false, false);
+      const auto y = __builtin_amdgcn_permlane16_swap(a.y, c.y, false, false);
+      const int dim = 16 * (d + (g & 1)) + 8 * (g >> 1);
+      if (ok && (16 * d + 32 <= DV || dim < DV))
+        *reinterpret_cast<uint4*>(row + dim) = make_uint4(x[0], y[0], x[1], y[1]);
+    }
+    if constexpr (kVS % 2 == 1) {
+      const uint2 a = packed(kVS - 1);
+      const int dim = 16 * (kVS - 1) + 4 * g;
+      if (ok && dim < DV) *reinterpret_cast<uint2*>(row + dim) = a;
+    }
+  };
+
   PageCache pc;
   // One query block of the work-group, start to finish: this half streams stages
   // [st_lo, st_hi) of it (st0: the block's first stage) and every wave passes
@@ -664,17 +651,23 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
                          static_cast<int64_t>(hq) * D;
 #pragma unroll
     for (int c = 0; c < kQC; ++c) {
-      const int d0 = kFp8T ? (D / 4) * g + 8 * c : 32 * c + 8 * g;
+      const int d0 = 32 * c + 8 * g;
       const uint4 v = (ok && d0 < D) ? *reinterpret_cast<const uint4*>(qp + d0)
                                      : make_uint4(0, 0, 0, 0);
       qb[nb][c] = __builtin_bit_cast(bf16x8_t, v);
     }
   }
-  // Running max per query column (log2 units, this lane's column r), and the
-  // softmax denominators in the O layout: l_acc[nb][i] is the sum for query row
-  // 4g + i, accumulated by an MFMA of P against ones beside the P.V ones (the
-  // same bf16 P weights as the numerator), so no VALU adds and no cross-lane
-  // fetch at the end.
+  // Running max per query column (log2 units, this lane's column r), and O^T: the
+  // P.V MFMAs take V^T as A and P^T as B, so column r of O is the same query as
+  // column r of S, and o[nb][d] holds its dims 16 d + 4 g .. + 3: the rescale and
+  // the final division need no value from another lane.  l_acc[nb]: the column's
+  // softmax denominator (four copies), accumulated by an MFMA of ones and P
+  // beside the P.V ones (the same bf16 P weights as the numerator).
+  // Against O with queries as rows (four ds_bpermute per rescale and merge, 64
+  // two-byte stores per block instead of 8 of 16 bytes): same box, A/B in
+  // alternating processes, two rounds, us: 1x2048 57.6 / 57.6 -> 55.0 / 55.1, 13
+  // ragged fp8 prompts 138.3 / 138.5 -> 136.0 / 136.0, ragged vision encoder
+  // 223.0 / 223.6 -> 218.8 / 219.2, 1x12288 1217 / 1204 -> 1210 / 1195.
   float m_run[kCB];
   // kFmaExp: the max the exponent subtracts, m_run once it is finite and kFar
   // before (so that the first visible score of a column exceeds it by more than
@@ -722,7 +715,7 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
   // Same box, A/B in alternating processes, two rounds (µs): 1x2048 60.3 / 59.6 ->
   // 59.6 / 59.0, 4x512 over 4096 161.9 / 160.2 -> 155.9 / 156.3, 16x512 75.6 / 76.1 ->
   // 74.2 / 74.5; at head size 64 (Whisper heads, 4x512 over 4096) 124.9 -> 128.1.
-  constexpr bool kVEarly = FK_PREFILL_VEARLY && !kFp8T && kDVP >= 128 && kDVP < 256;
+  constexpr bool kVEarly = FK_PREFILL_VEARLY && kDVP >= 128 && kDVP < 256;
   short4_t vpre_a[kVS], vpre_b[kVS];  // kVEarly: the pair's V slices, read with its scores
   // kKEarly: tile a's K chunks of an unmasked stage, read right after the barrier,
   // before the stage's staging loads are issued, so that the scalar work of the
@@ -732,14 +725,13 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
   // 70.1 / 70.0 -> 68.7 / 68.4; at head 128 level to 1% slower (16x512 73.2 / 72.5
   // -> 74.0 / 73.0), so not there, nor at the sizes not measured.
   constexpr bool kKEarly =
-      FK_PREFILL_KEARLY && !kFp8T && kStageTiles == 2 && (kDQ == 64 || kDQ == 256);
+      FK_PREFILL_KEARLY && kStageTiles == 2 && (kDQ == 64 || kDQ == 256);
   uint4 kpre[kQC];
   bool kpre_ok = false;  // wave-uniform: kpre holds this pair's tile a
   auto pair_scores = [&](auto masked, int tok0, const uint8_t* buf, int tt, bool ok_a,
                          bool ok_b, short4_t (&p_a)[kCB], short4_t (&p_b)[kCB],
                          auto early) __attribute__((always_inline)) {
     constexpr bool kMasked = decltype(masked)::value;
-    DTile<kFp8T, D> ta, tb;
     // Scores of tile a for every column block, then tile b's K is read: the two
     // K tiles are never live at once (20 fewer VGPRs in the compiler's own
     // allocation; measured 1% faster).
@@ -750,16 +742,11 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
     __builtin_amdgcn_s_setprio(1);
     {
       uint4 ka[kQC];
-      if constexpr (kFp8T) {
-        lds_tile_k<kFp8T, D>(buf, tt, r, g, ta);
-        k_chunks_d(ta, ka, ks);
-      } else {
-        if (kKEarly && kpre_ok) {
+      if (kKEarly && kpre_ok) {
 #pragma unroll
-          for (int c = 0; c < kQC; ++c) ka[c] = kpre[c];
-        } else {
-          lds_k_chunks<D, DV>(buf, tt, r, g, ka);
-        }
+        for (int c = 0; c < kQC; ++c) ka[c] = kpre[c];
+      } else {
+        lds_k_chunks<D, DV>(buf, tt, r, g, ka);
       }
 #pragma unroll
       for (int nb = 0; nb < kCB; ++nb) sc_a[nb] = qk_scores_n(ka, qb[nb]);
@@ -767,12 +754,7 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
     asm volatile("" ::: "memory");  // tile b's K reads stay after tile a's
     {
       uint4 kb[kQC];
-      if constexpr (kFp8T) {
-        lds_tile_k<kFp8T, D>(buf, tt + 1, r, g, tb);
-        k_chunks_d(tb, kb, ks);
-      } else {
-        lds_k_chunks<D, DV>(buf, tt + 1, r, g, kb);
-      }
+      lds_k_chunks<D, DV>(buf, tt + 1, r, g, kb);
 #pragma unroll
       for (int nb = 0; nb < kCB; ++nb) sc_b[nb] = qk_scores_n(kb, qb[nb]);
     }
@@ -844,12 +826,8 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
           m_ref[nb] = m_new == kNegInf ? kFar : m_new;
           if constexpr (kLse) l32[nb] *= alpha;
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const float a = row_from(alpha, g, i);
-#pragma unroll
-            for (int d = 0; d < kVS; ++d) o[nb][d][i] *= a;
-            l_acc[nb][i] *= a;
-          }
+          for (int d = 0; d < kVS; ++d) o[nb][d] *= alpha;
+          l_acc[nb] *= alpha;
 #pragma unroll
           for (int i = 0; i < 8; ++i)
             sm[i] = (kMasked && sm[i] == kNegInf) ? kNegInf
@@ -882,14 +860,10 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
         // 1 where the column's max stays (also -inf to -inf), 0 from -inf.
         const float alpha = m_new == m_run[nb] ? 1.f : __builtin_amdgcn_exp2f(m_run[nb] - m_new);
         m_run[nb] = m_new;
-        if constexpr (kLse) l32[nb] *= alpha;  // column layout, like alpha
+        if constexpr (kLse) l32[nb] *= alpha;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float a = row_from(alpha, g, i);
-#pragma unroll
-          for (int d = 0; d < kVS; ++d) o[nb][d][i] *= a;
-          l_acc[nb][i] *= a;
-        }
+        for (int d = 0; d < kVS; ++d) o[nb][d] *= alpha;
+        l_acc[nb] *= alpha;
       }
       // A column with no visible key yet (masked stages only) keeps m = -inf;
       // all its P are masked to 0.
@@ -916,7 +890,7 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
                      const short4_t (&p_a)[kCB], const short4_t (&p_b)[kCB],
                      auto early) __attribute__((always_inline)) {
     asm volatile("" ::: "memory");  // V reads stay after the score work
-    if constexpr (!kFp8T && kDVP >= 256) {
+    if constexpr (kDVP >= 256) {
       // bf16 at head size 256: the V slices go in two halves (read, mask, MFMAs),
       // so that half the V operands are live at once and two waves fit on a
       // SIMD; otherwise as below.
@@ -962,60 +936,44 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
             const uint2 va = __builtin_bit_cast(uint2, vba[d]), vb = __builtin_bit_cast(uint2, vbb[d]);
             const bf16x8_t v8 = __builtin_bit_cast(bf16x8_t, make_uint4(va.x, va.y, vb.x, vb.y));
             o[nb][hh * kDS + d] =
-                __builtin_amdgcn_mfma_f32_16x16x32_bf16(pab, v8, o[nb][hh * kDS + d], 0, 0, 0);
+                __builtin_amdgcn_mfma_f32_16x16x32_bf16(v8, pab, o[nb][hh * kDS + d], 0, 0, 0);
           }
           if (hh == 1)
-            l_acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pab, ones, l_acc[nb], 0, 0, 0);
+            l_acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pab, l_acc[nb], 0, 0, 0);
         }
         __builtin_amdgcn_s_setprio(0);
       }
       return;
     }
     short4_t vba[kVS], vbb[kVS];  // shared by the column blocks
-    if constexpr (!kFp8T) {
-      // Slice d holds dims 16d .. 16d + 15 (lane r: dim 16d + r).
+    // Slice d holds dims 16d .. 16d + 15 (lane r: dim 16d + r).
+#pragma unroll
+    for (int d = 0; d < kVS; ++d) {
+      if constexpr (kVEarly && decltype(early)::value) {
+        vba[d] = vpre_a[d];
+        vbb[d] = vpre_b[d];
+      } else {
+        lds_v_slice2<D, DV>(buf, tt, d, r, g, vba[d], vbb[d]);
+      }
+    }
+    // Zero the masked keys' V rows so that P = 0 never meets a NaN.
+    if (vmask) {
+      uint32_t ma[2], mb[2];
+#pragma unroll
+      for (int h2 = 0; h2 < 2; ++h2) {
+        const int k0 = tok0 + 4 * g + 2 * h2;
+        ma[h2] = ((ok_a && k0 < kend) ? 0x0000ffffu : 0u) | ((ok_a && k0 + 1 < kend) ? 0xffff0000u : 0u);
+        mb[h2] = ((ok_b && k0 + kTile < kend) ? 0x0000ffffu : 0u) |
+                 ((ok_b && k0 + kTile + 1 < kend) ? 0xffff0000u : 0u);
+      }
 #pragma unroll
       for (int d = 0; d < kVS; ++d) {
-        if constexpr (kVEarly && decltype(early)::value) {
-          vba[d] = vpre_a[d];
-          vbb[d] = vpre_b[d];
-        } else {
-          lds_v_slice2<D, DV>(buf, tt, d, r, g, vba[d], vbb[d]);
-        }
+        uint2 wa = __builtin_bit_cast(uint2, vba[d]), wb = __builtin_bit_cast(uint2, vbb[d]);
+        wa.x &= ma[0]; wa.y &= ma[1];
+        wb.x &= mb[0]; wb.y &= mb[1];
+        vba[d] = __builtin_bit_cast(short4_t, wa);
+        vbb[d] = __builtin_bit_cast(short4_t, wb);
       }
-      // Zero the masked keys' V rows so that P = 0 never meets a NaN.
-      if (vmask) {
-        uint32_t ma[2], mb[2];
-#pragma unroll
-        for (int h2 = 0; h2 < 2; ++h2) {
-          const int k0 = tok0 + 4 * g + 2 * h2;
-          ma[h2] = ((ok_a && k0 < kend) ? 0x0000ffffu : 0u) | ((ok_a && k0 + 1 < kend) ? 0xffff0000u : 0u);
-          mb[h2] = ((ok_b && k0 + kTile < kend) ? 0x0000ffffu : 0u) |
-                   ((ok_b && k0 + kTile + 1 < kend) ? 0xffff0000u : 0u);
-        }
-#pragma unroll
-        for (int d = 0; d < kVS; ++d) {
-          uint2 wa = __builtin_bit_cast(uint2, vba[d]), wb = __builtin_bit_cast(uint2, vbb[d]);
-          wa.x &= ma[0]; wa.y &= ma[1];
-          wb.x &= mb[0]; wb.y &= mb[1];
-          vba[d] = __builtin_bit_cast(short4_t, wa);
-          vbb[d] = __builtin_bit_cast(short4_t, wb);
-        }
-      }
-    } else {
-      // Slice d holds dims (D/16) r + d (lane r), packed from the row loads.
-      DTile<kFp8T, D> ta, tb;
-      lds_tile_v<kFp8T, D>(buf, tt, r, g, ta);
-      lds_tile_v<kFp8T, D>(buf, tt + 1, r, g, tb);
-      bool keep_a[4], keep_b[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        keep_a[i] = ok_a && tok0 + 4 * g + i < kend;
-        keep_b[i] = ok_b && tok0 + kTile + 4 * g + i < kend;
-      }
-      const bool vall = !vmask;
-      v_operands_fp8(ta, vsc, vall, keep_a, vba);
-      v_operands_fp8(tb, vsc, vall, keep_b, vbb);
     }
     __builtin_amdgcn_s_setprio(1);
     // P.V over the 32 keys with the 16x16x32 MFMA (the 16x16x16 one takes as
@@ -1034,9 +992,9 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
       for (int d = 0; d < kVS; ++d) {
         const uint2 va = __builtin_bit_cast(uint2, vba[d]), vb = __builtin_bit_cast(uint2, vbb[d]);
         const bf16x8_t v8 = __builtin_bit_cast(bf16x8_t, make_uint4(va.x, va.y, vb.x, vb.y));
-        o[nb][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pab, v8, o[nb][d], 0, 0, 0);
+        o[nb][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v8, pab, o[nb][d], 0, 0, 0);
       }
-      l_acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pab, ones, l_acc[nb], 0, 0, 0);
+      l_acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pab, l_acc[nb], 0, 0, 0);
     }
     __builtin_amdgcn_s_setprio(0);
   };
@@ -1295,15 +1253,6 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
 #pragma unroll
     for (int nb = 0; nb < kCB; ++nb) l32[nb] = pair_sum(l32[nb]);
   }
-  // Row maxima and sums of the rows this lane holds (row 4g + i of block nb).
-  float m_row[kCB][4], l_row[kCB][4];
-#pragma unroll
-  for (int nb = 0; nb < kCB; ++nb)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      m_row[nb][i] = row_from(m_run[nb], g, i);
-      l_row[nb][i] = l_acc[nb][i];
-    }
   if (kKS > 1 && !solo) {
 #pragma unroll 1
     for (int k = st_hi - st_lo; k < nsteps; ++k) {  // the shorter half's empty steps
@@ -1338,31 +1287,18 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
       for (int nb = 0; nb < kCB; ++nb) {
         const float mb_col = xm[nb * 64 + lane];
         const floatx4_t lb = *reinterpret_cast<const floatx4_t*>(xl + (nb * 64 + lane) * 4);
-        if constexpr (kLse) {  // the same merge for the columns' fp32 sums
-          const float ma = m_run[nb];
-          const float mx = fmaxf(ma, mb_col);
-          const float wa = ma == kNegInf ? 0.f : __builtin_amdgcn_exp2f(ma - mx);
-          const float wb = mb_col == kNegInf ? 0.f : __builtin_amdgcn_exp2f(mb_col - mx);
-          l32[nb] = l32[nb] * wa + x32[nb * 64 + lane] * wb;
-          m_run[nb] = mx;
-        }
-        float wa[4], wb[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float ma = m_row[nb][i];
-          const float mb = row_from(mb_col, g, i);
-          const float mx = fmaxf(ma, mb);
-          wa[i] = ma == kNegInf ? 0.f : __builtin_amdgcn_exp2f(ma - mx);
-          wb[i] = mb == kNegInf ? 0.f : __builtin_amdgcn_exp2f(mb - mx);
-          m_row[nb][i] = mx;
-          l_row[nb][i] = l_row[nb][i] * wa[i] + lb[i] * wb[i];
-        }
+        const float ma = m_run[nb];
+        const float mx = fmaxf(ma, mb_col);
+        const float wa = ma == kNegInf ? 0.f : __builtin_amdgcn_exp2f(ma - mx);
+        const float wb = mb_col == kNegInf ? 0.f : __builtin_amdgcn_exp2f(mb_col - mx);
+        if constexpr (kLse) l32[nb] = l32[nb] * wa + x32[nb * 64 + lane] * wb;
+        m_run[nb] = mx;
+        l_acc[nb] = l_acc[nb] * wa + lb * wb;
 #pragma unroll
         for (int d = 0; d < kVS; ++d) {
           const floatx4_t ob =
               *reinterpret_cast<const floatx4_t*>(xo + ((nb * kVS + d) * 64 + lane) * 4);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) o[nb][d][i] = o[nb][d][i] * wa[i] + ob[i] * wb[i];
+          o[nb][d] = o[nb][d] * wa + ob * wb;
         }
       }
     }
@@ -1380,86 +1316,36 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
         static_cast<uint8_t*>(P.part) + part_ml_offset(xs, P.part_rows, P.num_heads, DV));
 #pragma unroll
     for (int nb = 0; nb < kCB; ++nb) {
-      if constexpr (kLse) {  // column layout: lanes of row group 0 hold column r's sum
-        const int jc = j0 + 16 * nb + r;
-        if (g == 0 && jc < q_len)
-          part_ml[((prow0 + jc) * P.num_heads + hq) * kPartMl + 2] = l32[nb];
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int jr = j0 + 16 * nb + 4 * g + i;
-        if (jr >= q_len) continue;
-        const int64_t rh = (prow0 + jr) * P.num_heads + hq;
-        uint16_t* const po = part_o + rh * DV;
-#pragma unroll
-        for (int d = 0; d < kVS; ++d) {
-          const int dim = kFp8T ? (D / 16) * r + d : 16 * d + r;
-          if (kFp8T ? dim < DV : (16 * d + 16 <= DV || dim < DV))
-            po[dim] = __builtin_bit_cast(uint16_t, static_cast<__bf16>(o[nb][d][i]));
-        }
-        if (r == 0) {
-          float* const pm = part_ml + rh * kPartMl;
-          pm[0] = m_row[nb][i];
-          pm[1] = l_row[nb][i];
-        }
+      const int jr = j0 + 16 * nb + r;  // this lane's query
+      const int64_t rh = (prow0 + jr) * P.num_heads + hq;
+      write_row(part_o + rh * DV, o[nb], 1.f, jr < q_len);
+      if (g == 0 && jr < q_len) {
+        float* const pm = part_ml + rh * kPartMl;
+        pm[0] = m_run[nb];
+        pm[1] = l_acc[nb][0];
+        if constexpr (kLse) pm[2] = l32[nb];
       }
     }
     return;
   }
 
-  // kLse: lse = ln(sum e^(scale q.k)) = (m + log2 l) ln 2 per query column, the
-  // sink included; -inf for a row with no visible key.  Lanes of row group 0
-  // (r = column) write it.
-  if constexpr (kLse) {
-#pragma unroll
-    for (int nb = 0; nb < kCB; ++nb) {
-      const int jc = j0 + 16 * nb + r;
-      float l = l32[nb];
-      if (P.sinks) l = with_sink(l, m_run[nb], P.sinks[hq] * kLog2e);
-      if (g == 0 && jc < q_len)
-        P.lse[hq * P.lse_row_stride + q_start + jc] =
-            l > 0.f ? (m_run[nb] + __log2f(l)) * 0.6931471805599453f : kNegInf;
-    }
-  }
-
 #pragma unroll
   for (int nb = 0; nb < kCB; ++nb) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int jr = j0 + 16 * nb + 4 * g + i;  // query row this lane holds
-      float l = l_row[nb][i];
-      if (P.sinks) l = with_sink(l, m_row[nb][i], P.sinks[hq] * kLog2e);
-      if (jr >= q_len) continue;
-      const float f = l > 0.f ? 1.f / l : 0.f;
-      uint16_t* orow = P.out + static_cast<int64_t>(q_start + jr) * P.out_row_stride +
-                       static_cast<int64_t>(hq) * DV;
-      if constexpr (!kFp8T) {
-        // o[nb][d] holds dim 16d + r: lanes r = 0..15 write 16 adjacent dims (the
-        // padding dims past DV are not written).
-#pragma unroll
-        for (int d = 0; d < kVS; ++d)
-          if (16 * d + 16 <= DV || 16 * d + r < DV)
-            orow[16 * d + r] = __builtin_bit_cast(uint16_t, static_cast<__bf16>(o[nb][d][i] * f));
-      } else {
-        // o[nb][d] holds dim (D/16) r + d: D/16 adjacent dims per lane.
-        uint32_t w[D / 32];
-#pragma unroll
-        for (int d = 0; d < D / 32; ++d) {
-          const bf16x2_t pk = {static_cast<__bf16>(o[nb][2 * d][i] * f),
-                               static_cast<__bf16>(o[nb][2 * d + 1][i] * f)};
-          w[d] = __builtin_bit_cast(uint32_t, pk);
-        }
-        uint16_t* dst = orow + (D / 16) * r;
-        if constexpr (D == 64) {
-          *reinterpret_cast<uint2*>(dst) = make_uint2(w[0], w[1]);
-        } else {
-#pragma unroll
-          for (int q = 0; q < D / 128; ++q)
-            *reinterpret_cast<uint4*>(dst + 8 * q) =
-                make_uint4(w[4 * q], w[4 * q + 1], w[4 * q + 2], w[4 * q + 3]);
-        }
-      }
+    const int jr = j0 + 16 * nb + r;  // this lane's query
+    const float sink2 = P.sinks ? P.sinks[hq] * kLog2e : kNegInf;
+    // kLse: lse = ln(sum e^(scale q.k)) = (m + log2 l) ln 2 per query column, the
+    // sink included; -inf for a row with no visible key.  Lanes of row group 0
+    // write it.
+    if constexpr (kLse) {
+      const float ls = with_sink(l32[nb], m_run[nb], sink2);
+      if (g == 0 && jr < q_len)
+        P.lse[hq * P.lse_row_stride + q_start + jr] =
+            ls > 0.f ? (m_run[nb] + __log2f(ls)) * 0.6931471805599453f : kNegInf;
     }
+    const float l = with_sink(l_acc[nb][0], m_run[nb], sink2);
+    write_row(P.out + static_cast<int64_t>(q_start + jr) * P.out_row_stride +
+                  static_cast<int64_t>(hq) * DV,
+              o[nb], l > 0.f ? 1.f / l : 0.f, jr < q_len);
   }
   };
   const int heavy = nqb - 1 - x;
