@@ -42,6 +42,7 @@ struct PrefillShape {
   int ks;           // key parts within a work-group (1 or 2)
   int xs;           // key parts over work-groups (1: none), with a workspace
   int ks_plain;     // ks of the same call without a workspace (xs = 1)
+  bool part_f32;    // the key parts' O in fp32 rather than bf16
 };
 
 PrefillShape prefill_shape(bool paged, bool fp8, int64_t batch, int64_t max_seqlen_q,
@@ -63,6 +64,7 @@ PrefillShape prefill_shape(bool paged, bool fp8, int64_t batch, int64_t max_seql
   sh.ks = ((std::max(head_size, head_size_v) <= 192 || paged) && wgs < 2LL * num_cus()) ? 2 : 1;
   sh.ks_plain = sh.ks;
   sh.xs = 1;
+  sh.part_f32 = part_in_f32(head_size, head_size_v);
   const int64_t ncu = num_cus();
   // Where the key split would run (fewer 4-wave work-groups than two per CU):
   // 4-wave work-groups, two per CU, with each block's keys in xs parts over
@@ -140,7 +142,7 @@ PrefillShape prefill_shape(bool paged, bool fp8, int64_t batch, int64_t max_seql
 // Bytes of the work-group key split's partial states (0 without the split).
 int64_t prefill_ws_bytes(const PrefillShape& sh, int64_t total_q, int num_heads, int head_size_v) {
   if (sh.xs <= 1) return 0;
-  const int64_t bytes = part_ml_offset(sh.xs, total_q, num_heads, head_size_v) +
+  const int64_t bytes = part_ml_offset(sh.xs, total_q, num_heads, head_size_v, sh.part_f32) +
                         static_cast<int64_t>(sh.xs) * total_q * num_heads * kPartMl * 4;
   return (bytes + 255) / 256 * 256;
 }
@@ -166,6 +168,7 @@ struct PrefillMergeParams {
   int64_t lse_row_stride;
 };
 
+template <bool kF32>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillMergeParams M) {
   const int chunks = M.dv / 8;
   const int64_t t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
@@ -177,16 +180,23 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillMergeParams M
   const int hq = static_cast<int>(rh - row * M.num_heads);
   const int64_t plane = M.part_rows * M.num_heads;  // (row, head) records per part
   const float* const ml = reinterpret_cast<const float*>(
-      static_cast<const uint8_t*>(M.part) + part_ml_offset(M.xs, M.part_rows, M.num_heads, M.dv));
-  const uint16_t* const po = static_cast<const uint16_t*>(M.part);
-  // Every part's record and O slice (8 bf16) are loaded before any is used.
+      static_cast<const uint8_t*>(M.part) + part_ml_offset(M.xs, M.part_rows, M.num_heads, M.dv, kF32));
+  const uint8_t* const po = static_cast<const uint8_t*>(M.part);
+  // Every part's record and O slice (8 values) are loaded before any is used.
   float4 rec[kMaxKeyParts];
   uint4 ov[kMaxKeyParts];
+  float4 of[kF32 ? kMaxKeyParts : 1][2];
 #pragma unroll
   for (int p = 0; p < kMaxKeyParts; ++p) {
     if (p < M.xs) {
       rec[p] = *reinterpret_cast<const float4*>(ml + (p * plane + rh) * kPartMl);
-      ov[p] = *reinterpret_cast<const uint4*>(po + (p * plane + rh) * M.dv + 8 * c8);
+      const int64_t at = (p * plane + rh) * M.dv + 8 * c8;
+      if constexpr (kF32) {
+        of[p][0] = *reinterpret_cast<const float4*>(po + at * 4);
+        of[p][1] = *reinterpret_cast<const float4*>(po + at * 4 + 16);
+      } else {
+        ov[p] = *reinterpret_cast<const uint4*>(po + at * 2);
+      }
     }
   }
   float mx = kNegInf;
@@ -200,11 +210,18 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillMergeParams M
       const float w = rec[p].x == kNegInf ? 0.f : __builtin_amdgcn_exp2f(rec[p].x - mx);
       l += w * rec[p].y;
       l32 += w * rec[p].z;
-      const uint32_t ow[4] = {ov[p].x, ov[p].y, ov[p].z, ov[p].w};
+      if constexpr (kF32) {
+        const float x[8] = {of[p][0].x, of[p][0].y, of[p][0].z, of[p][0].w,
+                            of[p][1].x, of[p][1].y, of[p][1].z, of[p][1].w};
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {  // dims 2i (low half) and 2i + 1 (high half)
-        acc[2 * i] += w * __builtin_bit_cast(float, ow[i] << 16);
-        acc[2 * i + 1] += w * __builtin_bit_cast(float, ow[i] & 0xffff0000u);
+        for (int i = 0; i < 8; ++i) acc[i] += w * x[i];
+      } else {
+        const uint32_t ow[4] = {ov[p].x, ov[p].y, ov[p].z, ov[p].w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {  // dims 2i (low half) and 2i + 1 (high half)
+          acc[2 * i] += w * __builtin_bit_cast(float, ow[i] << 16);
+          acc[2 * i + 1] += w * __builtin_bit_cast(float, ow[i] & 0xffff0000u);
+        }
       }
     }
   }
@@ -368,9 +385,11 @@ int prefill_entry(const char* name, bool paged, void* out, int64_t out_row_strid
     M.lse = lse;
     M.lse_row_stride = lse_row_stride;
     const int64_t threads = total_q * num_heads * (head_size_v / 8);
-    if (threads > 0)
-      hipLaunchKernelGGL(prefill_merge_kernel, dim3(static_cast<unsigned>((threads + 255) / 256)),
-                         dim3(256), 0, s, M);
+    const dim3 mgrid(static_cast<unsigned>((threads + 255) / 256));
+    if (threads > 0 && sh.part_f32)
+      hipLaunchKernelGGL(prefill_merge_kernel<true>, mgrid, dim3(256), 0, s, M);
+    else if (threads > 0)
+      hipLaunchKernelGGL(prefill_merge_kernel<false>, mgrid, dim3(256), 0, s, M);
   }
   return check_launch(name);
 }

@@ -87,11 +87,11 @@ struct PrefillParams {
   int64_t lse_row_stride;
   // Work-group key split: each query block's key stages are divided over xs
   // work-groups (1: none), which leave their partial states in `part` for
-  // prefill_merge_kernel: O [xs][part_rows][num_heads][DV] bf16 (before the
-  // division by the sum, rounded once), then from byte 2 xs part_rows num_heads
-  // DV (a multiple of 16: DV is a multiple of 8) [xs][part_rows][num_heads][4]
-  // fp32 (running max in log2 units, the sum the output divides by, the fp32 sum
-  // of the log-sum-exp output, unused).
+  // prefill_merge_kernel: O [xs][part_rows][num_heads][DV] before the division by
+  // the sum, in bf16 (rounded once) or fp32 (part_in_f32), then (a multiple of 16
+  // bytes on: DV is a multiple of 8) [xs][part_rows][num_heads][4] fp32 (running
+  // max in log2 units, the sum the output divides by, the fp32 sum of the
+  // log-sum-exp output, unused).
   int xs;
   void* part;
   int64_t part_rows;  // rows of q (at least cu_seqlens_q[batch])
@@ -105,10 +105,15 @@ struct PrefillParams {
 
 // Floats of the partial state per (part, row, head) besides O.
 constexpr int kPartMl = 4;
-// The fp32 records of the key parts' states, after their bf16 O.
+// MLA's head sizes keep the key parts' O in fp32: with 128 query tokens a
+// work-group (two column blocks) they take parts at sizes that ran whole with 64,
+// and against 64-bit results the error of bf16 parts was 3.3e-3 there, of whole
+// blocks and of fp32 parts 2.9e-3.
+constexpr bool part_in_f32(int D, int DV) { return D > 128 && DV <= 128; }
+// The fp32 records of the key parts' states, after their O.
 __host__ __device__ inline int64_t part_ml_offset(int xs, int64_t part_rows, int num_heads,
-                                                  int dv) {
-  return static_cast<int64_t>(xs) * part_rows * num_heads * dv * 2;
+                                                  int dv, bool part_f32) {
+  return static_cast<int64_t>(xs) * part_rows * num_heads * dv * (part_f32 ? 4 : 2);
 }
 constexpr int kMaxKeyParts = 8;  // work-group key split: parts per query block at most
 
@@ -126,8 +131,9 @@ namespace {
 // Two waves per SIMD (two 4-wave work-groups per CU; each holds 32 KB of LDS for
 // bf16 pages at head size 128, 64 KB at 256).  At 256 the bf16 P.V operands go
 // in two halves to fit in the 256 registers two waves leave (fp8 fits as is);
-// dense keys at 256 (the row clamping) would still spill 11 VGPRs, so one.
-constexpr int prefill_waves_per_simd(int D, bool paged) { return D > 192 && !paged ? 1 : 2; }
+// dense keys fit since their row clamping works on 32-bit offsets (one wave
+// before: 2 x (1500 .. 2500) tokens at 8 heads of 256, not causal, 219 -> 140 us).
+constexpr int kPrefillWavesPerSimd = 2;
 #ifndef FK_PREFILL_LAZY
 #define FK_PREFILL_LAZY 8.0f
 #endif
@@ -142,9 +148,12 @@ constexpr bool kFmaExp = FK_PREFILL_FMA_EXP;
 constexpr float kFar = -1.0e30f;  // the max the exponent subtracts before a column's first key
 constexpr int kQTokens = 16 * kColBlocks;      // query tokens per wave at head size 128
 // Column blocks per wave at head sizes (D, DV): at 256 the O accumulators of one
-// block (16 tiles of 4 fp32 per lane) already take what two take at 128; above
-// 128 the query operands and key tiles of two blocks would not fit beside them.
-constexpr int col_blocks_for(int D, int DV) { return (D > 128 || DV > 128) ? 1 : kColBlocks; }
+// block (16 tiles of 4 fp32 per lane) already take what two take at 128.  MLA's
+// 192 / 128 takes two (246 registers): each K / V byte read from LDS then serves
+// 32 queries, and a work-group 128 instead of 64.  Same box, us: 877 and 1200 new
+// tokens over 2669 and 3300 cached ones, 16 heads (both calls and the merge) 249
+// -> 206; 300 .. 2000 over 500 .. 1500 178 -> 160; 1x256 over 8192 unchanged (64).
+constexpr int col_blocks_for(int D, int DV) { return (D > 192 || DV > 128) ? 1 : kColBlocks; }
 // MFMA extents: the score MFMAs run over D rounded up to 32, P.V over DV rounded
 // up to 16.
 constexpr int qk_extent(int D) { return (D + 31) / 32 * 32; }
@@ -273,16 +282,8 @@ struct Stage {
 // buffer is read).  M0 carries the LDS address: an input operand bound to M0, so
 // the compiler writes it (and knows it changed) with no save and restore; the
 // s_nop is the wait state between that write and the load that reads M0.
-__device__ __forceinline__ void lds_dma16(const uint8_t* src, uint32_t lds_addr) {
-  asm volatile(
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %0, off"
-      :
-      : "v"(src), "{m0}"(lds_addr)
-      : "memory");
-}
-// The same load with a wave-uniform 64-bit base in SGPRs and a per-lane 32-bit
-// byte offset (the load's saddr form): lane l reads base + off.  A tile's base
+// The address is a wave-uniform 64-bit base in SGPRs and a per-lane 32-bit byte
+// offset (the load's saddr form): lane l reads base + off.  A tile's base
 // changes from stage to stage and the lanes' offsets do not, so a stage's
 // loads take no 64-bit address arithmetic per lane.
 __device__ __forceinline__ void lds_dma16_s(const uint8_t* base, uint32_t off, uint32_t lds_addr) {
@@ -418,7 +419,7 @@ __device__ __forceinline__ bool lpt_item(const PrefillParams& P, const int32_t* 
 // fp32 sum of P per query column besides (8 adds per column block and 32 keys).
 template <bool kFp8, bool kPaged, int D, int DV, int kKS, bool kLse = false>
 __global__ __launch_bounds__(kKS * kPrefillWaves * 64)
-__attribute__((amdgpu_waves_per_eu(prefill_waves_per_simd(D > DV ? D : DV, kPaged)))) void
+__attribute__((amdgpu_waves_per_eu(kPrefillWavesPerSimd))) void
 paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
                      const int32_t* __restrict__ cu_q, const int32_t* __restrict__ cu_k) {
   static_assert(!kFp8 || (D == DV && (D == 64 || D == 128 || D == 256)),
@@ -715,7 +716,7 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
   // Same box, A/B in alternating processes, two rounds (µs): 1x2048 60.3 / 59.6 ->
   // 59.6 / 59.0, 4x512 over 4096 161.9 / 160.2 -> 155.9 / 156.3, 16x512 75.6 / 76.1 ->
   // 74.2 / 74.5; at head size 64 (Whisper heads, 4x512 over 4096) 124.9 -> 128.1.
-  constexpr bool kVEarly = FK_PREFILL_VEARLY && kDVP >= 128 && kDVP < 256;
+  constexpr bool kVEarly = FK_PREFILL_VEARLY && kDVP >= 128 && kDVP < 256 && kDQ <= 128;
   short4_t vpre_a[kVS], vpre_b[kVS];  // kVEarly: the pair's V slices, read with its scores
   // kKEarly: tile a's K chunks of an unmasked stage, read right after the barrier,
   // before the stage's staging loads are issued, so that the scalar work of the
@@ -1068,7 +1069,7 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
         vt[tt] = pc.vb + slot * static_cast<uint32_t>(P.v_row_bytes);
         row0[tt] = 0;
       } else {
-        row0[tt] = static_cast<int64_t>(k_start) + tok;
+        row0[tt] = min(static_cast<int64_t>(k_start) + tok, row_cap);
         kt[tt] = kh + row0[tt] * P.k_row_bytes;
         vt[tt] = vh + row0[tt] * P.v_row_bytes;
       }
@@ -1087,17 +1088,22 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
           base = which ? vt[u] : kt[u];
           first = row0[u];
         }
-      if (kPaged || first + 15 <= row_cap) {
+      if (kPaged || row_cap - first >= 15) {
         // (padded rows: the padding chunks are not loaded)
         if ((S::kKReal == S::kKChunks && S::kVReal == S::kVChunks) || lane_ld[i])
           lds_dma16_s(base, lane_off[i], buf_addr + 16 * pos0);
       } else {
-        // Dense keys whose tile runs past the tensor's end: clamp each row.
+        // Dense keys whose tile runs past the sequence's last row: the rows past it
+        // read that row (their 32-bit offset taken back by the rows they are past
+        // it; 64-bit row addresses here took 10 to 20 registers more in every dense
+        // kernel, at heads of 72 and 80 the third wave per SIMD: ragged vision
+        // encoder, 16 heads of 80, 219 -> 184.5 us, 1x3000 99.5 -> 72.7).
         int wh, row, q;
         slot_of(i, wh, row, q);
-        const int64_t rb = which ? P.v_row_bytes : P.k_row_bytes;
-        const uint8_t* src = (which ? vh : kh) + min(first + (row & 15), row_cap) * rb + 16 * q;
-        if (lane_ld[i]) lds_dma16(src, buf_addr + 16 * pos0);
+        const int past = max(0, (row & 15) - static_cast<int>(row_cap - first));
+        const uint32_t rb = static_cast<uint32_t>(which ? P.v_row_bytes : P.k_row_bytes);
+        if (lane_ld[i])
+          lds_dma16_s(base, lane_off[i] - static_cast<uint32_t>(past) * rb, buf_addr + 16 * pos0);
       }
     }
   };
@@ -1291,14 +1297,17 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
         const float mx = fmaxf(ma, mb_col);
         const float wa = ma == kNegInf ? 0.f : __builtin_amdgcn_exp2f(ma - mx);
         const float wb = mb_col == kNegInf ? 0.f : __builtin_amdgcn_exp2f(mb_col - mx);
-        if constexpr (kLse) l32[nb] = l32[nb] * wa + x32[nb * 64 + lane] * wb;
+        // (Explicit FMAs: every variant of the kernel rounds alike.)
+        if constexpr (kLse)
+          l32[nb] = __builtin_fmaf(x32[nb * 64 + lane], wb, l32[nb] * wa);
         m_run[nb] = mx;
-        l_acc[nb] = l_acc[nb] * wa + lb * wb;
+        l_acc[nb][0] = __builtin_fmaf(lb[0], wb, l_acc[nb][0] * wa);
 #pragma unroll
         for (int d = 0; d < kVS; ++d) {
           const floatx4_t ob =
               *reinterpret_cast<const floatx4_t*>(xo + ((nb * kVS + d) * 64 + lane) * 4);
-          o[nb][d] = o[nb][d] * wa + ob * wb;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[nb][d][i] = __builtin_fmaf(ob[i], wb, o[nb][d][i] * wa);
         }
       }
     }
@@ -1311,14 +1320,21 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
   // one that saw no key (max -inf, sum 0).
   if (xs > 1) {
     const int64_t prow0 = static_cast<int64_t>(xpart) * P.part_rows + q_start;
-    uint16_t* const part_o = static_cast<uint16_t*>(P.part);
     float* const part_ml = reinterpret_cast<float*>(
-        static_cast<uint8_t*>(P.part) + part_ml_offset(xs, P.part_rows, P.num_heads, DV));
+        static_cast<uint8_t*>(P.part) + part_ml_offset(xs, P.part_rows, P.num_heads, DV, part_in_f32(D, DV)));
 #pragma unroll
     for (int nb = 0; nb < kCB; ++nb) {
       const int jr = j0 + 16 * nb + r;  // this lane's query
       const int64_t rh = (prow0 + jr) * P.num_heads + hq;
-      write_row(part_o + rh * DV, o[nb], 1.f, jr < q_len);
+      if constexpr (part_in_f32(D, DV)) {
+        float* const po = static_cast<float*>(P.part) + rh * DV;
+#pragma unroll
+        for (int d = 0; d < kVS; ++d)
+          if (jr < q_len && (16 * d + 16 <= DV || 16 * d + 4 * g < DV))
+            *reinterpret_cast<floatx4_t*>(po + 16 * d + 4 * g) = o[nb][d];
+      } else {
+        write_row(static_cast<uint16_t*>(P.part) + rh * DV, o[nb], 1.f, jr < q_len);
+      }
       if (g == 0 && jr < q_len) {
         float* const pm = part_ml + rh * kPartMl;
         pm[0] = m_run[nb];
