@@ -73,6 +73,14 @@ __device__ __forceinline__ uint2 fp8x4_to_bf16x4(uint32_t w, float s) {
   return make_uint2(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b));
 }
 
+// 4 OCP e4m3fn bytes -> 4 bf16 of the same values (exact: the scaled conversion
+// with a scale of one, two elements an instruction).
+__device__ __forceinline__ uint2 fp8x4_to_bf16x4_exact(uint32_t w) {
+  return make_uint2(
+      __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.f, false)),
+      __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.f, true)));
+}
+
 // KV loads (plain cached loads: marking them non-temporal measured slower).
 __device__ __forceinline__ uint4 ld16(const uint8_t* p) { return *reinterpret_cast<const uint4*>(p); }
 __device__ __forceinline__ uint2 ld8(const uint8_t* p) { return *reinterpret_cast<const uint2*>(p); }

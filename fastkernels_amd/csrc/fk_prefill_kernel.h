@@ -15,8 +15,7 @@
 // [k_len - q_len + j - window_left, k_len - q_len + j].  A query with no
 // visible key gets a zero row.  Attention sinks (s_aux: one logit per query
 // head) join each row's softmax denominator, as in the decode kernel.  kv head
-// = hq / (Hq / Hk); fp8 pages are dequantised per kv head as in the decode
-// kernel.  Optionally the kernel also writes each row's softmax log-sum-exp,
+// = hq / (Hq / Hk); fp8 pages are dequantised per kv head.  Optionally the kernel also writes each row's softmax log-sum-exp,
 // lse = ln(sum_k e^(scale q.k)) (flash_attn_varlen_func's return_softmax_lse,
 // fastkernels/tasks/baseline/L1/flash_attn_varlen.py:33-46; -inf for a row
 // with no visible key), fp32 [Hq, total_q] with a row stride.
@@ -426,9 +425,9 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
                 "fp8 pages: equal query / value head sizes 64, 128 or 256");
   using S = Stage<kFp8, D, DV>;
   // fp8 pages: the work-group converts each staged stage once into a bf16
-  // stage (float(x) * scale rounded to bf16, the value each wave would form),
-  // and the waves compute on bf16 tiles, instead of each wave dequantising the
-  // same K / V bytes for its own query head.  Up to head size 128 each fp8
+  // stage (exactly: the scales are applied to the scores and the rows), and the
+  // waves compute on bf16 tiles, instead of each wave converting the same K / V
+  // bytes for its own query head.  Up to head size 128 each fp8
   // buffer has its bf16 one (kConv); at 256 two of those would not fit in LDS
   // with two work-groups per CU, so one bf16 buffer serves the stages in turn
   // (kConv1: converted after every wave is done with the stage before, a second
@@ -543,10 +542,16 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
                                  : nullptr;
   // Dense keys: rows past the sequence's last key would run off the tensor.
   const int64_t row_cap = kPaged ? INT64_MAX : static_cast<int64_t>(k_start) + max(k_len, 1) - 1;
-  const float s2 = P.scale_log2;
-  // fp8 dequant scales of kv head h (1 for bf16 pages or no scale tensor): each
-  // K / V element enters the MFMAs as float(x) * scale rounded to bf16.
-  const float ks = (kFp8 && P.k_scale) ? P.k_scale[h] : 1.f;
+  // fp8 dequant scales of kv head h (1 for bf16 pages or no scale tensor), one per
+  // head: every e4m3fn value is a bf16 value, so K and V enter the MFMAs exactly
+  // and K's scale joins the softmax scale, V's the division by the row sum (no
+  // rounding of float(x) * scale to bf16; error against 64-bit results 3.0e-3 ->
+  // 2.1e-3).  Same box, A/B in alternating processes, us, against float(x) * scale
+  // rounded to bf16 per element (two products and a rounding per two elements more):
+  // 13 ragged prompts 136.0 -> 132.0, 1x2048 65.4 -> 63.3, 4x512 over 4096 227 ->
+  // 206, 1x512 over 8192 115.6 -> 106.1, 16 / 2 / 256 457 -> 402, 64 / 8 / 64 351
+  // -> 331.
+  const float s2 = (kFp8 && P.k_scale) ? P.scale_log2 * P.k_scale[h] : P.scale_log2;
   const float vsc = (kFp8 && P.v_scale) ? P.v_scale[h] : 1.f;
 
   const int win = P.window_left;
@@ -1185,9 +1190,8 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
         const int row = rem / S::kKChunks;
         const int q = rem - row * S::kKChunks;
         const uint4 x = *reinterpret_cast<const uint4*>(fbuf + S::offset(which, row, q));
-        const float sc = which ? vsc : ks;
-        const uint2 a = fp8x4_to_bf16x4(x.x, sc), b = fp8x4_to_bf16x4(x.y, sc);
-        const uint2 e = fp8x4_to_bf16x4(x.z, sc), f = fp8x4_to_bf16x4(x.w, sc);
+        const uint2 a = fp8x4_to_bf16x4_exact(x.x), b = fp8x4_to_bf16x4_exact(x.y);
+        const uint2 e = fp8x4_to_bf16x4_exact(x.z), f = fp8x4_to_bf16x4_exact(x.w);
         *reinterpret_cast<uint4*>(bbuf + SB::offset(which, row, 2 * q)) = make_uint4(a.x, a.y, b.x, b.y);
         *reinterpret_cast<uint4*>(bbuf + SB::offset(which, row, 2 * q + 1)) =
             make_uint4(e.x, e.y, f.x, f.y);
@@ -1333,7 +1337,7 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
           if (jr < q_len && (16 * d + 16 <= DV || 16 * d + 4 * g < DV))
             *reinterpret_cast<floatx4_t*>(po + 16 * d + 4 * g) = o[nb][d];
       } else {
-        write_row(static_cast<uint16_t*>(P.part) + rh * DV, o[nb], 1.f, jr < q_len);
+        write_row(static_cast<uint16_t*>(P.part) + rh * DV, o[nb], vsc, jr < q_len);
       }
       if (g == 0 && jr < q_len) {
         float* const pm = part_ml + rh * kPartMl;
@@ -1361,7 +1365,7 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
     const float l = with_sink(l_acc[nb][0], m_run[nb], sink2);
     write_row(P.out + static_cast<int64_t>(q_start + jr) * P.out_row_stride +
                   static_cast<int64_t>(hq) * DV,
-              o[nb], l > 0.f ? 1.f / l : 0.f, jr < q_len);
+              o[nb], l > 0.f ? vsc / l : 0.f, jr < q_len);
   }
   };
   const int heavy = nqb - 1 - x;
