@@ -61,21 +61,9 @@ __device__ __forceinline__ uint32_t hi_pair(uint32_t a, uint32_t b) {
   return __builtin_amdgcn_perm(b, a, 0x07060302u);  // (a >> 16) | (b & 0xffff0000)
 }
 
-// 4 OCP e4m3fn bytes -> 4 bf16 holding float(x) * s rounded to nearest even:
-// the per-tensor fp8 dequant of _cast_kv_tile (triton_unified_attention.py:
-// 64-67), (data.to(float32) * scale).to(q.dtype).  With s = 1 it is exact (every
-// e4m3fn value is a bf16 value).
-__device__ __forceinline__ uint2 fp8x4_to_bf16x4(uint32_t w, float s) {
-  const auto lo = __builtin_amdgcn_cvt_pk_f32_fp8(w, false);
-  const auto hi = __builtin_amdgcn_cvt_pk_f32_fp8(w, true);
-  const bf16x2_t a = {static_cast<__bf16>(lo[0] * s), static_cast<__bf16>(lo[1] * s)};
-  const bf16x2_t b = {static_cast<__bf16>(hi[0] * s), static_cast<__bf16>(hi[1] * s)};
-  return make_uint2(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b));
-}
-
 // 4 OCP e4m3fn bytes -> 4 bf16 of the same values (exact: the scaled conversion
 // with a scale of one, two elements an instruction).
-__device__ __forceinline__ uint2 fp8x4_to_bf16x4_exact(uint32_t w) {
+__device__ __forceinline__ uint2 fp8x4_to_bf16x4(uint32_t w) {
   return make_uint2(
       __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.f, false)),
       __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.f, true)));
@@ -195,10 +183,9 @@ struct DTile {
 };
 
 // K operand chunks (bf16, dims as described at DTile) of a loaded tile; fp8
-// bytes are dequantised with scale s (fp8x4_to_bf16x4).
+// bytes are converted exactly (fp8x4_to_bf16x4).
 template <bool kFp8, int D>
-__device__ __forceinline__ void k_chunks_d(const DTile<kFp8, D>& t, uint4 (&kc)[D / 32],
-                                           float s = 1.f) {
+__device__ __forceinline__ void k_chunks_d(const DTile<kFp8, D>& t, uint4 (&kc)[D / 32]) {
   if constexpr (!kFp8) {
 #pragma unroll
     for (int c = 0; c < D / 32; ++c) kc[c] = t.k[c];
@@ -209,71 +196,38 @@ __device__ __forceinline__ void k_chunks_d(const DTile<kFp8, D>& t, uint4 (&kc)[
       const uint4& src = t.k[c >> 1];
       const uint32_t w0 = (c & 1) ? src.z : src.x;
       const uint32_t w1 = (c & 1) ? src.w : src.y;
-      const uint2 lo = fp8x4_to_bf16x4(w0, s), hi = fp8x4_to_bf16x4(w1, s);
+      const uint2 lo = fp8x4_to_bf16x4(w0), hi = fp8x4_to_bf16x4(w1);
       kc[c] = make_uint4(lo.x, lo.y, hi.x, hi.y);
     }
   }
 }
 
-// V row i of a loaded tile as D/32 words of bf16 pairs (zero when !keep); fp8
-// bytes are dequantised with scale s.
-template <bool kFp8, int D>
-__device__ __forceinline__ void v_words(const DTile<kFp8, D>& t, int i, bool keep,
-                                        uint32_t (&w)[D / 32], float s = 1.f) {
-  if constexpr (!kFp8) {
+// V row i of a loaded bf16 tile as D/32 words of pairs (zero when !keep).
+template <int D>
+__device__ __forceinline__ void v_words(const DTile<false, D>& t, int i, bool keep,
+                                        uint32_t (&w)[D / 32]) {
 #pragma unroll
-    for (int q = 0; q < D / 32; ++q) w[q] = keep ? t.v[i][q] : 0u;
-  } else {
-#pragma unroll
-    for (int q = 0; q < D / 64; ++q) {
-      const uint2 x = fp8x4_to_bf16x4(t.v[i][q], s);
-      w[2 * q] = keep ? x.x : 0u;
-      w[2 * q + 1] = keep ? x.y : 0u;
-    }
-  }
+  for (int q = 0; q < D / 32; ++q) w[q] = keep ? t.v[i][q] : 0u;
 }
 
-// P.V B operands straight from the fp8 V rows of a loaded tile: slice d takes
-// dim (D/16) r + d of rows 4g .. 4g+3, each float(x) * s rounded to bf16 (the
-// dequant of fp8x4_to_bf16x4).  The rounding instruction packs two rows' values
-// of one dim, so the pairs come out in operand order with no byte regrouping
-// (v_words + v_operands_w pack two dims of one row, then permute).  Unless
-// `all`, the bytes of row i are zeroed where !keep[i] (a NaN byte becomes 0).
+// P.V B operands from the fp8 V rows of a loaded tile: slice d takes dim
+// (D/16) r + d of rows 4g .. 4g+3, converted exactly.  The conversion packs two
+// dims of one row; v_operands_w then pairs the rows.  Unless `all`, the bytes of
+// row i are zeroed where !keep[i] (a NaN byte becomes 0).
 template <int D>
-__device__ __forceinline__ void v_operands_fp8(const DTile<true, D>& t, float s, bool all,
+__device__ __forceinline__ void v_operands_fp8(const DTile<true, D>& t, bool all,
                                                const bool (&keep)[4], short4_t (&vb)[D / 16]) {
   constexpr int NW = D / 64;  // fp8 words per row: dims 4q .. 4q + 3 in word q
-  uint32_t w[4][NW];
+  uint32_t vw[4][2 * NW];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int q = 0; q < NW; ++q) w[i][q] = t.v[i][q];
-  if (!all) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int q = 0; q < NW; ++q) w[i][q] = keep[i] ? w[i][q] : 0u;
-  }
-#pragma unroll
-  for (int q = 0; q < NW; ++q) {
-    float f[4][4];  // [row][dim 4q + e]
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const auto lo = __builtin_amdgcn_cvt_pk_f32_fp8(w[i][q], false);
-      const auto hi = __builtin_amdgcn_cvt_pk_f32_fp8(w[i][q], true);
-      f[i][0] = lo[0] * s;
-      f[i][1] = lo[1] * s;
-      f[i][2] = hi[0] * s;
-      f[i][3] = hi[1] * s;
+    for (int q = 0; q < NW; ++q) {
+      const uint2 x = fp8x4_to_bf16x4(all || keep[i] ? t.v[i][q] : 0u);
+      vw[i][2 * q] = x.x;
+      vw[i][2 * q + 1] = x.y;
     }
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const bf16x2_t a = {static_cast<__bf16>(f[0][e]), static_cast<__bf16>(f[1][e])};
-      const bf16x2_t b = {static_cast<__bf16>(f[2][e]), static_cast<__bf16>(f[3][e])};
-      vb[4 * q + e] = __builtin_bit_cast(
-          short4_t, make_uint2(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b)));
-    }
-  }
+  v_operands_w(vw, vb);
 }
 
 }  // namespace fk

@@ -20,9 +20,10 @@
 // (triton_unified_attention.py:741-776): M = max m_s, L = sum l_s e^(m_s - M),
 // O = sum o_s e^(m_s - M) / L, and O = 0 when L = 0.  fp8 KV pages are
 // dequantised per kv head as float(x) * scale, the per-tensor rule of
-// _cast_kv_tile (triton_unified_attention.py:51-67): each K and V element is
-// float(x) * scale rounded to bf16 before it enters the MFMAs, as the reference
-// casts the scaled tile to the query dtype.
+// _cast_kv_tile (triton_unified_attention.py:51-67).  Every e4m3fn value is a
+// bf16 value, so K and V enter the MFMAs exactly; K's scale joins the softmax
+// scale and V's the row's normalisation (the reference rounds the scaled element
+// to the query dtype, an error this does not add).
 // Head sizes D = 64, 128 and 256 (the reference builds FlashAttnDecode at 128,
 // and at 256 and 64 for Qwen3-Next and Whisper, L2/qwen3_next_attention.py:
 // 148-150, L2/whisper_attention.py:185-190) are template instantiations.
@@ -396,10 +397,9 @@ struct WaveState {
         qb[c] = __builtin_bit_cast(bf16x8_t, v);
       }
     }
-    const float s2 = P.scale_log2;
-    // fp8 dequant scales of this kv head (1 for bf16 pages or no scale tensor).
-    const float ks = (kFp8 && P.k_scale) ? P.k_scale[kvh] : 1.f;
-    const float vsc = (kFp8 && P.v_scale) ? P.v_scale[kvh] : 1.f;
+    // K's fp8 dequant scale (one per kv head) joins the softmax scale; V's is
+    // applied when the rows are written (v_scale_of).
+    const float s2 = (kFp8 && P.k_scale) ? P.scale_log2 * P.k_scale[kvh] : P.scale_log2;
 
     m_run = kNegInf;
     l_run = 0.f;
@@ -479,7 +479,7 @@ struct WaveState {
         return;
       }
       uint4 kc[kKc];
-      k_chunks_d(cur, kc, ks);
+      k_chunks_d(cur, kc);
       const floatx4_t acc = qk_scores_n(kc, qb);
       // A tile wholly inside the visible keys on a readable page (every tile but
       // those at a segment's edges) needs no mask: one wave-uniform test skips
@@ -526,7 +526,7 @@ struct WaveState {
         bool keep[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) keep[i] = page >= 0 && static_cast<uint32_t>(rel0 + i) < span;
-        v_operands_fp8(cur, vsc, full, keep, vb);
+        v_operands_fp8(cur, full, keep, vb);
       } else {
         uint32_t vw[4][D / 32];
 #pragma unroll
@@ -677,9 +677,15 @@ struct WaveState {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the ring is free for the next segment
   }
 
+  // V's fp8 dequant scale of kv head kvh (1 for bf16 pages or no scale tensor).
+  __device__ __forceinline__ static float v_scale_of(const DecodeParams& P, int kvh) {
+    return (kFp8 && P.v_scale) ? P.v_scale[kvh] : 1.f;
+  }
+
   // Normalised output rows of the virtual head for a sequence finished in place.
   __device__ __forceinline__ void write_final(const DecodeParams& P, int b, const VHead& vh,
                                               int r, int g) const {
+    const float vsc = v_scale_of(P, vh.kvh);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int j = 4 * g + i;
@@ -688,7 +694,7 @@ struct WaveState {
         l = with_sink(l, row_value<kG>(m_run, g, i),
                       sink_log2(P, vh.qbase + (j < vh.ncols ? j : 0)));
       if (j >= kG || j >= vh.ncols) continue;
-      const float f = l > 0.f ? 1.f / l : 0.f;
+      const float f = l > 0.f ? vsc / l : 0.f;
       uint32_t w[D / 32];
 #pragma unroll
       for (int d = 0; d < D / 32; ++d) {
@@ -713,6 +719,7 @@ struct WaveState {
   // the virtual head's query heads hq.
   __device__ __forceinline__ void write_partial(const DecodeParams& P, int64_t row0,
                                                 const VHead& vh, int r, int g) const {
+    const float vsc = v_scale_of(P, vh.kvh);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int j = 4 * g + i;
@@ -721,7 +728,9 @@ struct WaveState {
 #pragma unroll
       for (int q = 0; q < kSl / 4; ++q)
         *reinterpret_cast<float4*>(dst + 4 * q) =
-            make_float4(o[4 * q][i], o[4 * q + 1][i], o[4 * q + 2][i], o[4 * q + 3][i]);
+            kFp8 ? make_float4(o[4 * q][i] * vsc, o[4 * q + 1][i] * vsc, o[4 * q + 2][i] * vsc,
+                               o[4 * q + 3][i] * vsc)
+                 : make_float4(o[4 * q][i], o[4 * q + 1][i], o[4 * q + 2][i], o[4 * q + 3][i]);
     }
     if (g == 0 && r < vh.ncols) {
       P.part_ml[(row0 + vh.qbase + r) * 2 + 0] = m_run;

@@ -1190,8 +1190,8 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
         const int row = rem / S::kKChunks;
         const int q = rem - row * S::kKChunks;
         const uint4 x = *reinterpret_cast<const uint4*>(fbuf + S::offset(which, row, q));
-        const uint2 a = fp8x4_to_bf16x4_exact(x.x), b = fp8x4_to_bf16x4_exact(x.y);
-        const uint2 e = fp8x4_to_bf16x4_exact(x.z), f = fp8x4_to_bf16x4_exact(x.w);
+        const uint2 a = fp8x4_to_bf16x4(x.x), b = fp8x4_to_bf16x4(x.y);
+        const uint2 e = fp8x4_to_bf16x4(x.z), f = fp8x4_to_bf16x4(x.w);
         *reinterpret_cast<uint4*>(bbuf + SB::offset(which, row, 2 * q)) = make_uint4(a.x, a.y, b.x, b.y);
         *reinterpret_cast<uint4*>(bbuf + SB::offset(which, row, 2 * q + 1)) =
             make_uint4(e.x, e.y, f.x, f.y);
