@@ -121,10 +121,14 @@ struct DecodeParams {
   int64_t new_k_stride;  // bytes between the rows of new_k
   int64_t new_v_stride;
   int slot_is_i64;
-  // Fixed partitions: waves per virtual head (1 or 2).  With 2, each takes half
-  // of the partition's tiles and the second leaves its state in LDS for the
-  // first to merge (launches that would otherwise leave one wave per SIMD).
+  // Fixed partitions: waves per virtual head (1, 2, 4 or 8).  Each takes a share
+  // of the partition's tiles and all but the first leave their state in LDS for
+  // the first to merge (launches that would otherwise leave one wave per SIMD,
+  // and whole windows, below).
   int split;
+  // Whole windows: one partition per sequence (max_parts 1), no merge launch; the
+  // partition kernel also zeroes the rows of sequences without context.
+  int solo;
 };
 
 // The query heads one wave handles: kv head kvh, query heads qbase .. qbase +
@@ -739,6 +743,13 @@ struct WaveState {
   }
 };
 
+// Zero row of D bf16 for an empty sequence (one wave; each lane D / 64 dims).
+template <int D>
+__device__ __forceinline__ void zero_row(uint16_t* orow, int lane) {
+#pragma unroll
+  for (int e = 0; e < D / 64; ++e) orow[(D / 64) * lane + e] = 0;
+}
+
 // Registers held to what two waves per SIMD leave (256 VGPRs + AGPRs): for a
 // work-group of fewer than 8 waves the compiler's own occupancy target would
 // let them grow past it (to 272 at head size 256, one wave per SIMD), and the
@@ -759,20 +770,20 @@ struct WaveState {
 // Fixed partitions: work-group = (partition p, virtual-head group, sequence b);
 // wave w owns virtual head blockIdx.y * NH + w and streams the partition.
 // Partial rows: (b * max_parts + p) * Hq + hq.
-// With P.split = 2 the work-group has 2 NH waves: wave w + NH takes the second
-// half of the partition's tiles for the same virtual head, leaves (O, max, sum)
-// in LDS (dynamic, split_state_floats per virtual head) and wave w merges it
-// with the log-sum-exp rule before writing.  A launch whose fixed partitions
+// With P.split = S > 1 the work-group has S NH waves: wave w + u NH takes the
+// u-th share of the partition's tiles for the same virtual head, leaves (O, max,
+// sum) in LDS (dynamic, split_state_floats per virtual head and share after the
+// first) and wave w merges them with the log-sum-exp rule before writing.  A launch whose fixed partitions
 // give one wave per SIMD (C5's 16 partitions: 8 sequences x 16 partitions x 8
 // kv heads = 1024 waves) then runs two.
 template <int D>
 constexpr int split_state_floats() { return (D / 16) * 4 * 64 + 2 * 64; }
 template <int NH, int kG, int D, bool kFp8, int U, bool kStore>
-__global__ __launch_bounds__(NH < 8 ? 2 * NH * 64 : NH * 64)
+__global__ __launch_bounds__(8 * 64)
 __attribute__((amdgpu_waves_per_eu(FK_DECODE_WAVES_PER_EU))) void paged_decode_partition_kernel(
     DecodeParams P, const int32_t* __restrict__ block_tables, const int32_t* __restrict__ ctx_lens,
     const void* __restrict__ slot_mapping) {
-  extern __shared__ __align__(16) float split_x[];  // P.split == 2: the second waves' states
+  extern __shared__ __align__(16) float split_x[];  // P.split > 1: the later shares' states
   const int p = blockIdx.x;
   const int b = blockIdx.z;
   const int ctx = ctx_lens[b];
@@ -780,7 +791,7 @@ __attribute__((amdgpu_waves_per_eu(FK_DECODE_WAVES_PER_EU))) void paged_decode_p
   // Wave index made provably uniform so that page lookups are scalar loads.
   const int wave_id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wave = wave_id & (NH - 1);  // the virtual-head slot
-  const int sub = wave_id / NH;         // which half of the partition (P.split == 2)
+  const int sub = wave_id / NH;         // which share of the partition (P.split > 1)
   const int v = blockIdx.y * NH + wave;
   // Waves past the last virtual head only keep the work-group's barrier count.
   const bool idle = v >= P.num_kv_heads * P.col_blocks;  // uniform over the wave
@@ -806,41 +817,49 @@ __attribute__((amdgpu_waves_per_eu(FK_DECODE_WAVES_PER_EU))) void paged_decode_p
     if (P.split == 1) {
       st.run(P, block_tables, slot_mapping, b, vh, seg_begin, tok_end, ctx, lo, r, g, idle);
     } else {
-      // Halves of the partition's tiles (the first takes the odd one); the
-      // waves stream different lengths, so no lock-step barriers.
+      // Shares of the partition's tiles (the first ones take one more); the waves
+      // stream different lengths, so no lock-step barriers.
       const int n = max(0, (tok_end - seg_begin + kTile - 1) / kTile);
-      const int mid = min(tok_end, seg_begin + ((n + 1) / 2) * kTile);
-      st.run(P, block_tables, slot_mapping, b, vh, sub == 0 ? seg_begin : mid,
-             sub == 0 ? mid : tok_end, ctx, lo, r, g, idle, false);
+      const int per = n / P.split;
+      const int more = n - per * P.split;
+      const int s0 = per * sub + min(sub, more);
+      const int s1 = s0 + per + (sub < more ? 1 : 0);
+      st.run(P, block_tables, slot_mapping, b, vh, min(tok_end, seg_begin + s0 * kTile),
+             min(tok_end, seg_begin + s1 * kTile), ctx, lo, r, g, idle, false);
       constexpr int kSl = D / 16;
       float* const x = split_x + wave * split_state_floats<D>();
-      if (sub == 1 && !idle) {
+      if (sub > 0 && !idle) {
+        float* const xs = x + (sub - 1) * NH * split_state_floats<D>();
 #pragma unroll
         for (int d = 0; d < kSl; ++d)
-          *reinterpret_cast<floatx4_t*>(x + (d * 64 + lane) * 4) = st.o[d];
-        x[kSl * 256 + lane] = st.m_run;
-        x[kSl * 256 + 64 + lane] = st.l_run;
+          *reinterpret_cast<floatx4_t*>(xs + (d * 64 + lane) * 4) = st.o[d];
+        xs[kSl * 256 + lane] = st.m_run;
+        xs[kSl * 256 + 64 + lane] = st.l_run;
       }
       __syncthreads();
-      if (sub == 1) return;
+      if (sub > 0) return;
       if (!idle) {
         // reduce_segments' rule per query column (m, l in column layout; O rows
         // 4g + i take their column's weights): M = max, w = 2^(m - M), 0 for an
-        // empty half.
-        const float mb = x[kSl * 256 + lane];
-        const float lb = x[kSl * 256 + 64 + lane];
-        const float ma = st.m_run;
-        const float mx = fmaxf(ma, mb);
-        const float wa = ma == kNegInf ? 0.f : __builtin_amdgcn_exp2f(ma - mx);
-        const float wb = mb == kNegInf ? 0.f : __builtin_amdgcn_exp2f(mb - mx);
-        st.m_run = mx;
-        st.l_run = st.l_run * wa + lb * wb;
+        // empty share.
+#pragma unroll 1
+        for (int u = 1; u < P.split; ++u) {
+          const float* const xs = x + (u - 1) * NH * split_state_floats<D>();
+          const float mb = xs[kSl * 256 + lane];
+          const float lb = xs[kSl * 256 + 64 + lane];
+          const float ma = st.m_run;
+          const float mx = fmaxf(ma, mb);
+          const float wa = ma == kNegInf ? 0.f : __builtin_amdgcn_exp2f(ma - mx);
+          const float wb = mb == kNegInf ? 0.f : __builtin_amdgcn_exp2f(mb - mx);
+          st.m_run = mx;
+          st.l_run = st.l_run * wa + lb * wb;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float fa = row_value<kG>(wa, g, i), fb = row_value<kG>(wb, g, i);
+          for (int i = 0; i < 4; ++i) {
+            const float fa = row_value<kG>(wa, g, i), fb = row_value<kG>(wb, g, i);
 #pragma unroll
-          for (int d = 0; d < kSl; ++d)
-            st.o[d][i] = st.o[d][i] * fa + x[(d * 64 + lane) * 4 + i] * fb;
+            for (int d = 0; d < kSl; ++d)
+              st.o[d][i] = st.o[d][i] * fa + xs[(d * 64 + lane) * 4 + i] * fb;
+          }
         }
       }
     }
@@ -851,6 +870,10 @@ __attribute__((amdgpu_waves_per_eu(FK_DECODE_WAVES_PER_EU))) void paged_decode_p
       const int64_t row0 = (static_cast<int64_t>(b) * P.max_parts + p) * P.num_heads;
       st.write_partial(P, row0, vh, r, g);
     }
+  }
+  if (P.solo && ctx <= 0 && !idle && sub == 0) {
+    for (int j = 0; j < vh.ncols; ++j)
+      zero_row<D>(P.out + b * P.out_row_stride + static_cast<int64_t>(vh.qbase + j) * D, lane);
   }
   // No partition streams position ctx - 1 (no context): partition 0 writes b's
   // row.
@@ -1163,13 +1186,6 @@ __device__ __forceinline__ void merge_group(const DecodeParams& P, uint16_t* out
   merge_write<D>(out_b + static_cast<int64_t>(hq) * D, out, sink_log2(P, hq), lane);
 }
 
-// Zero row of D bf16 for an empty sequence (one wave; each lane D / 64 dims).
-template <int D>
-__device__ __forceinline__ void zero_row(uint16_t* orow, int lane) {
-#pragma unroll
-  for (int e = 0; e < D / 64; ++e) orow[(D / 64) * lane + e] = 0;
-}
-
 // Fixed partitions: merge sequences with more than one partition; zero empty ones.
 // Work-group = kRows query heads blockIdx.x * kRows .. of sequence blockIdx.y
 // (merge_group).
@@ -1304,6 +1320,37 @@ int validate(const char* name, int64_t batch, int num_heads, int num_kv_heads, i
   return FK_OK;
 }
 
+// Whole windows.  Under a sliding window a sequence streams at most
+// (window_left + 16) / 16 + 1 tiles, whatever its context, so a batch can give
+// each sequence to one work-group, each virtual head's tiles in `shares` (1, 2, 4
+// or 8) over as many waves that merge in LDS, with no merge launch.  The fewest
+// shares are taken that fill the chip (kSoloWaves waves) with at most kSoloTiles
+// tiles a wave; where even the most do not fill it, they still run when a wave
+// has at most kSoloShort tiles (the balanced schedule's two launches cost more
+// than such a chain).  Returns 0 for the balanced schedule, which also evens out
+// long windows that only some of the sequences fill.  Kernel times on one box,
+// us, balanced (with its merge) -> whole windows, contexts 300 .. 6000: 64 / 8 / 64
+// heads, window 128, batch 16 12.5 -> 7.4, 128 29 -> 14, 256 55 -> 18; 32 / 8 / 128,
+// window 1024, batch 32 30.4 -> 24.5, 64 48.2 -> 45.5, window 512, batch 128 53.1
+// -> 45.
+constexpr int64_t kSoloWaves = 1024;
+constexpr int kSoloTiles = 9, kSoloShort = 3;
+constexpr size_t kSoloLds = 64 * 1024;
+size_t solo_lds(int nh, int shares, int head_size) {
+  return static_cast<size_t>(shares - 1) * nh * (head_size / 16 * 4 * 64 + 2 * 64) *
+         sizeof(float);
+}
+int solo_shares(int64_t batch, int vheads, int head_size, int window_left) {
+  if (window_left < 0 || window_left > (1 << 20)) return 0;
+  const int tiles = (window_left + kTile) / kTile + 1;
+  int most = 1;
+  for (int s = 1; s <= kMaxWavesPerGroup && solo_lds(1, s, head_size) <= kSoloLds; s *= 2) {
+    if (batch * vheads * s >= kSoloWaves && tiles <= s * kSoloTiles) return s;
+    most = s;
+  }
+  return tiles <= most * kSoloShort ? most : 0;
+}
+
 struct Launch {
   DecodeParams P;
   const void* slot_mapping = nullptr;
@@ -1403,6 +1450,23 @@ int prepare(const char* name, Launch& L, void* out, int64_t out_row_stride, cons
   // Fixed partitions that would run one wave per SIMD (or fewer) split each
   // partition over two waves of the work-group.
   P.split = 1;
+  P.solo = 0;
+  if (const int s = balanced ? solo_shares(batch, vh, head_size, window_left) : 0) {
+    L.balanced = false;
+    P.solo = 1;
+    P.part_tokens = 1 << 30;
+    P.max_parts = 1;
+    P.split = s;
+    // Work-groups of 8 waves or fewer whose states fit in 64 KB of LDS.
+    int nh = 1;
+    while (2 * nh * s <= kMaxWavesPerGroup && 2 * nh <= vh &&
+           solo_lds(2 * nh, s, head_size) <= kSoloLds)
+      nh *= 2;
+    L.nh = nh;
+    L.part_lds = solo_lds(nh, s, head_size);
+    L.grid = dim3(1, static_cast<unsigned>((vh + nh - 1) / nh), static_cast<unsigned>(batch));
+    return FK_OK;
+  }
   if (!balanced && L.nh <= 4 &&
       static_cast<int64_t>(max_parts) * batch * vh < 2LL * 4 * num_cus()) {
     P.split = 2;
@@ -1591,6 +1655,7 @@ extern "C" int fk_paged_decode_reduce(
                    batch, num_heads, num_kv_heads, head_size, block_size, num_blocks, scale,
                    window_left, sinks, part_tokens, max_parts, workspace, ws_bytes);
   if (rc != FK_OK || batch == 0) return rc;
+  if (L.P.solo) return FK_OK;  // whole windows: nothing to merge
   hipStream_t s = as_stream(stream);
   switch (head_size) {
     case 64: launch_reduce_d<64>(L, batch, num_heads, s); break;

@@ -1,0 +1,79 @@
+"""Sliding-window decode launches that give a sequence's whole window to one work-group
+(its waves merge in LDS, no merge launch) against the fixed partitions over the same
+inputs, at the edges of the rule that picks them: one sequence, as many as fill the chip,
+windows of one token up to a wave's most tiles, every head size and query group, fp8
+pages, empty contexts, masked pages, and the fused store.
+
+Both paths sum in fp32 and round P and the row to bf16, so they differ by the rounding of
+P (2^-9 relative each) and of the result: rtol = 2^-7, and atol = 2^-7 of values of N(0, 1)
+rows averaged over the window."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from fastkernels_amd import ops, workloads
+
+pytestmark = pytest.mark.gpu
+
+# (batch, query heads, kv heads, head size, window_left, fp8)
+CASES = [
+    (1, 64, 8, 64, 127, False),
+    (1, 32, 8, 128, 0, False),
+    (3, 32, 8, 128, 368, False),    # 24 tiles: the most a few sequences take
+    (5, 16, 2, 256, 176, False),    # 12 tiles, head 256 (at most 4 shares)
+    (40, 64, 8, 64, 128, False),
+    (150, 32, 8, 128, 127, True),   # one share per head
+    (17, 71, 1, 64, 500, False),    # several column blocks per kv head
+    (33, 20, 20, 64, 1136, False),  # 72 tiles over 8 shares
+    (130, 8, 1, 128, 300, True),
+    (2, 40, 1, 256, 15, True),
+]
+
+
+@pytest.mark.parametrize("batch,hq,hk,d,window,fp8", CASES)
+def test_whole_windows_match_partitions(cuda, batch, hq, hk, d, window, fp8):
+    print(f"windows {batch} {hq}/{hk}/{d} {window} fp8={fp8}", flush=True)
+    lens = [(977 * i * i + 31 * i) % 1500 for i in range(batch)]  # 0 first, then mixed
+    if batch == 1:
+        lens = [1203]
+    pool = sum((n + 15) // 16 for n in lens) + 2
+    make = workloads.c5_fp8_decode if fp8 else workloads.c3_decode
+    case = make(cuda, num_heads=hq, kv_heads=hk, head_dim=d, block_size=16, pool_blocks=pool,
+                ctx_lens=lens, seed=batch + window)
+    bt = case.block_tables.clone()
+    if batch > 2:  # a page inside the last sequences' windows that must not be read
+        rows = [b for b in range(batch) if lens[b] > 40][-2:]
+        for b in rows:
+            bt[b, (lens[b] - 20) // 16] = -1
+    sinks = torch.linspace(-3, 3, hq, device=cuda)
+    outs = []
+    for splits in (0, 4):
+        part, parts, nbytes = ops.paged_decode_plan(batch, hq, hk, d, max(lens), splits)
+        ws = torch.zeros(max(1, nbytes), dtype=torch.uint8, device=cuda)
+        out = torch.full_like(case.q, float("nan"))
+        ops.paged_decode(out, case.q, case.k_cache, case.v_cache, bt, case.ctx_lens, case.scale,
+                         part, parts, ws, case.k_scale, case.v_scale, window, sinks)
+        torch.cuda.synchronize()
+        outs.append(out.float())
+    assert torch.isfinite(outs[0]).all()
+    torch.testing.assert_close(outs[0], outs[1], rtol=2 ** -7, atol=2 ** -7)
+    for b in range(batch):
+        if lens[b] == 0:
+            assert not outs[0][b].any()
+    # The fused store: the same bits as the store, then the decode.
+    rows = workloads.decode_step_rows(case)
+    kc, vc = case.k_cache.clone(), case.v_cache.clone()
+    ops.store_kvcache(rows.key, rows.value, kc, vc, rows.slot_mapping)
+    part, parts, nbytes = ops.paged_decode_plan(batch, hq, hk, d, max(lens), 0)
+    ws = torch.zeros(max(1, nbytes), dtype=torch.uint8, device=cuda)
+    want, got = torch.empty_like(case.q), torch.empty_like(case.q)
+    ops.paged_decode(want, case.q, kc, vc, case.block_tables, case.ctx_lens, case.scale, part,
+                     parts, ws, case.k_scale, case.v_scale, window, sinks)
+    ops.store_paged_decode(got, case.q, rows.key, rows.value, case.k_cache, case.v_cache,
+                           rows.slot_mapping, case.block_tables, case.ctx_lens, case.scale, part,
+                           parts, ws, case.k_scale, case.v_scale, window, sinks)
+    torch.cuda.synchronize()
+    assert bool(torch.equal(want.view(torch.int16), got.view(torch.int16)))
+    assert bool(torch.equal(kc.view(torch.uint8), case.k_cache.view(torch.uint8)))
+    assert bool(torch.equal(vc.view(torch.uint8), case.v_cache.view(torch.uint8)))
