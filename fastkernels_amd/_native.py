@@ -45,8 +45,7 @@ _SIGNATURES = {
                                      c_void_p, c_int, c_int64, c_int, c_int, c_int, c_int,
                                      c_int64, c_void_p]),
     "fk_paged_decode_plan": (c_int, [c_int64, c_int, c_int, c_int, c_int64, c_int,
-                                     ctypes.POINTER(c_int64), ctypes.POINTER(c_int64),
-                                     ctypes.POINTER(c_int64)]),
+                                     c_void_p, c_void_p, c_void_p]),
     "fk_paged_decode": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_int,
                                 c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_int,
                                 c_int, c_int, c_int, c_int64, c_float, c_int, c_void_p,
@@ -152,7 +151,9 @@ def check(fn: str, code: int) -> None:
 
 def call(fn: str, *args) -> None:
     """Call entry point ``fn`` and raise FkError on a non-zero status."""
-    check(fn, getattr(lib(), fn)(*args))
+    rc = getattr(_lib or lib(), fn)(*args)
+    if rc != FK_OK:
+        check(fn, rc)
 
 
 def prefill_split_bytes(paged: bool, kv_dtype: int, batch: int, total_q: int, max_seqlen_q: int,
@@ -172,11 +173,7 @@ def plan(batch: int, num_heads: int, num_kv_heads: int, head_size: int, max_seq_
          num_splits: int) -> tuple[int, int, int]:
     """fk_paged_decode_plan: (part_tokens, max_parts, workspace_bytes); part_tokens 0 is
     the length-balanced schedule."""
-    part = c_int64(0)
-    nparts = c_int64(0)
-    ws = c_int64(0)
-    check("fk_paged_decode_plan",
-          lib().fk_paged_decode_plan(batch, num_heads, num_kv_heads, head_size, max_seq_len,
-                                     num_splits, ctypes.byref(part), ctypes.byref(nparts),
-                                     ctypes.byref(ws)))
-    return part.value, nparts.value, ws.value
+    out = (c_int64 * 3)()
+    call("fk_paged_decode_plan", batch, num_heads, num_kv_heads, head_size, max_seq_len, num_splits,
+         ctypes.byref(out), ctypes.byref(out, 8), ctypes.byref(out, 16))
+    return tuple(out)

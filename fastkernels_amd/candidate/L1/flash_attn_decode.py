@@ -162,7 +162,9 @@ class FlashAttnDecode(nn.Module):
             return None
         if not isinstance(s, torch.Tensor):
             s = torch.tensor([float(s)], dtype=torch.float32)
-        s = s.to(device=device, dtype=torch.float32).reshape(-1)
+        if s.dtype != torch.float32 or s.device != device:
+            s = s.to(device=device, dtype=torch.float32)
+        s = s.reshape(-1)
         if s.numel() == 1:
             s = s.expand(hk)
         if s.numel() != hk:
@@ -171,19 +173,23 @@ class FlashAttnDecode(nn.Module):
 
     def _launch_args(self, q, k_cache, cache_seqlens, kwargs):
         """Parses the reference's decode kwargs; returns what both launch paths need."""
-        max_seq_len = kwargs.pop("max_seq_len", None)
-        block_table = kwargs.pop("block_table", None)
-        softmax_scale = kwargs.pop("softmax_scale", None)
-        kwargs.pop("causal", None)
-        num_splits = int(kwargs.pop("num_splits", 0) or 0)
-        out = kwargs.pop("out", None)
-        k_scale = kwargs.pop("k_scale", kwargs.pop("k_descale", None))
-        v_scale = kwargs.pop("v_scale", kwargs.pop("v_descale", None))
-        window = kwargs.pop("window_size", None)
+        pop = kwargs.pop
+        max_seq_len = pop("max_seq_len", None)
+        block_table = pop("block_table", None)
+        softmax_scale = pop("softmax_scale", None)
+        pop("causal", None)
+        num_splits = out = k_scale = v_scale = window = s_aux = None
+        if kwargs:
+            num_splits = pop("num_splits", None)
+            out = pop("out", None)
+            k_scale = pop("k_scale", pop("k_descale", None))
+            v_scale = pop("v_scale", pop("v_descale", None))
+            window = pop("window_size", None)
+            s_aux = pop("s_aux", None)
+            pop("scheduler_metadata", None)
+        num_splits = int(num_splits or 0)
         if window is None:
             window = self._window_size
-        s_aux = kwargs.pop("s_aux", None)
-        kwargs.pop("scheduler_metadata", None)
         # A decode query is the last token, so only the left extent matters.
         window_left = int(window[0]) if window is not None and int(window[0]) >= 0 else -1
         if kwargs:
@@ -210,17 +216,22 @@ class FlashAttnDecode(nn.Module):
                                      num_splits)
         ws = self._get_workspace(plan.workspace_bytes, q.device)
         if out is None:
-            out = torch.empty((b, self.num_heads, self.head_dim), dtype=q.dtype, device=q.device)
+            out = q.new_empty((b, self.num_heads, self.head_dim))
         return dict(out=out, block_table=block_table, cache_seqlens=cache_seqlens,
                     softmax_scale=float(softmax_scale), part_tokens=plan.part_tokens,
                     max_parts=plan.max_parts, ws=ws, k_scale=k_scale, v_scale=v_scale,
                     window_left=window_left, sinks=sinks)
 
+    def _heads(self, t: torch.Tensor, b: int) -> torch.Tensor:
+        """t as [b, num_heads, head_dim]."""
+        shape = (b, self.num_heads, self.head_dim)
+        return t if t.shape == shape else t.view(shape)
+
     def forward(self, q, k_cache, v_cache, cache_seqlens=None, **kwargs):
         a = self._launch_args(q, k_cache, cache_seqlens, kwargs)
         b = q.shape[0]
-        q3 = q.view(b, self.num_heads, self.head_dim)
-        out3 = a["out"].view(b, self.num_heads, self.head_dim)
+        q3 = self._heads(q, b)
+        out3 = self._heads(a["out"], b)
         call = torch.ops.fastkernels_amd.paged_decode if torch.compiler.is_compiling() \
             else ops.paged_decode
         call(out3, q3, k_cache, v_cache, a["block_table"], a["cache_seqlens"], a["softmax_scale"],

@@ -48,14 +48,15 @@ class RMSNorm(nn.Module):
     def forward(self, x: torch.Tensor, residual: torch.Tensor | None = None):
         weight = self.weight if self.elementwise_affine else self._unit_weight
         if weight.dtype != x.dtype or weight.device != x.device:
-            weight = weight.to(device=x.device, dtype=x.dtype)
-        weight = weight.detach()
+            weight = weight.detach().to(device=x.device, dtype=x.dtype)
         if x.stride(-1) != 1 or not self._rows_view_ok(x):
             # e.g. the per-head q/k norm of Qwen3 on a [N, H, D] view of the fused
             # qkv buffer: the reference makes such inputs contiguous too
             # (rms_norm.py forward_cuda).
             x = x.contiguous()
         compiling = torch.compiler.is_compiling()
+        if compiling:
+            weight = weight.detach()
         if residual is None:
             out = torch.empty_like(x, memory_format=torch.contiguous_format)
             if compiling:

@@ -71,6 +71,14 @@ class RotaryEmbedding(nn.Module):
             cache = cache.to(query.dtype)
         return cache
 
+    @staticmethod
+    def _norm_weight(norm: nn.Module, query: torch.Tensor) -> torch.Tensor:
+        """The norm's weight, contiguous, on the query's device in its dtype."""
+        w = norm.weight if norm.elementwise_affine else norm._unit_weight
+        if torch.compiler.is_compiling() or w.dtype != query.dtype or w.device != query.device:
+            w = w.detach().to(device=query.device, dtype=query.dtype)
+        return w.contiguous()
+
     def forward_store(self, positions: torch.Tensor, query: torch.Tensor, key: torch.Tensor,
                       value: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
                       slot_mapping: torch.Tensor, q_norm: nn.Module | None = None,
@@ -88,17 +96,18 @@ class RotaryEmbedding(nn.Module):
             if q_norm.eps != k_norm.eps:
                 raise ValueError("RotaryEmbedding.forward_store: q_norm and k_norm eps differ")
             eps = q_norm.eps
-            qw = (q_norm.weight if q_norm.elementwise_affine else q_norm._unit_weight).detach()
-            kw = (k_norm.weight if k_norm.elementwise_affine else k_norm._unit_weight).detach()
-            qw = qw.to(device=query.device, dtype=query.dtype).contiguous()
-            kw = kw.to(device=query.device, dtype=query.dtype).contiguous()
+            qw = self._norm_weight(q_norm, query)
+            kw = self._norm_weight(k_norm, query)
         cache = self._cache_for(query)
         if positions.dtype != torch.int64:
             positions = positions.to(torch.int64)
         if not positions.is_contiguous():
             positions = positions.contiguous()
-        k3 = k_cache.view(k_cache.shape[0], k_cache.shape[1], -1, self.head_dim)
-        v3 = v_cache.view(v_cache.shape[0], v_cache.shape[1], -1, self.head_dim)
+        k3, v3 = k_cache, v_cache
+        if k_cache.dim() != 4 or k_cache.shape[3] != self.head_dim:
+            k3 = k_cache.view(k_cache.shape[0], k_cache.shape[1], -1, self.head_dim)
+        if v_cache.dim() != 4 or v_cache.shape[3] != self.head_dim:
+            v3 = v_cache.view(v_cache.shape[0], v_cache.shape[1], -1, self.head_dim)
         if k_cache.dtype != query.dtype:
             # A cache of another dtype (fp8): the fused kernel stores bit copies, so
             # run the ops one by one, the store converting as tl.store does.

@@ -27,7 +27,7 @@ class SiluAndMul(nn.Module):
         d = x.shape[-1] // 2
         if x.stride(-1) != 1:
             x = x.contiguous()
-        out = torch.empty(x.shape[:-1] + (d,), dtype=x.dtype, device=x.device)
+        out = x.new_empty(x.shape[:-1] + (d,))
         if torch.compiler.is_compiling():
             torch.ops.fastkernels_amd.silu_and_mul(out, x)
         else:

@@ -14,7 +14,6 @@ stay opaque under torch.compile and are capturable in HIP graphs.
 from __future__ import annotations
 
 import math
-from ctypes import c_void_p
 from typing import NamedTuple
 
 import torch
@@ -36,18 +35,27 @@ def _tag(t: torch.Tensor, what: str) -> int:
         raise TypeError(f"{what}: unsupported dtype {t.dtype}") from None
 
 
-def _stream(t: torch.Tensor) -> c_void_p:
-    if t.device.type != "cuda":
+# The checks below run on every call of kernels that take a few µs, so they read each
+# tensor's sizes and strides once, compare device indices, and make views only for the
+# layouts that need one (a decode step of one sequence, four operators: 77 -> 49 µs of
+# host time, 17 of them the six launches).
+def _stream(t: torch.Tensor) -> int:
+    if not t.is_cuda:
         raise RuntimeError(f"fastkernels_amd ops run on the GPU only (got a {t.device} tensor)")
-    return c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
-def _ptr(t: torch.Tensor | None) -> c_void_p:
-    return c_void_p(t.data_ptr() if t is not None else 0)
+def _ptr(t: torch.Tensor | None) -> int | None:
+    return None if t is None else t.data_ptr()
 
 
 def _rows(t: torch.Tensor, width: int, what: str) -> tuple[int, int]:
     """(rows, row_stride) of a tensor viewed as [rows, width] with unit inner stride."""
+    if t.dim() == 2:
+        n, w = t.shape
+        s0, s1 = t.stride()
+        if w == width and s1 == 1 and n > 0 and w > 0:
+            return n, (s0 if n > 1 else width)  # (one row: its stride is never used)
     if t.dim() == 0:
         raise ValueError(f"{what}: expected at least one dimension")
     if t.numel() == 0:
@@ -65,11 +73,11 @@ def _rows(t: torch.Tensor, width: int, what: str) -> tuple[int, int]:
     return v.shape[0], v.stride(0)
 
 
-def _same_device(*ts: torch.Tensor) -> None:
-    dev = ts[0].device
-    for t in ts[1:]:
-        if t is not None and t.device != dev:
-            raise ValueError(f"tensors on different devices: {dev} vs {t.device}")
+def _same_device(first: torch.Tensor, *ts: torch.Tensor | None) -> None:
+    dev = first.get_device()
+    for t in ts:
+        if t is not None and t.get_device() != dev:
+            raise ValueError(f"tensors on different devices: {first.device} vs {t.device}")
 
 
 # ---------------------------------------------------------------------------
@@ -128,29 +136,11 @@ def rotary_embedding(positions: torch.Tensor, query: torch.Tensor, key: torch.Te
         raise TypeError("rotary_embedding: query and key must share a dtype")
     if tokens == 0:
         return
-    qw = query.numel() // tokens
-    if qw % head_size:
-        raise ValueError("rotary_embedding: query width is not a multiple of head_size")
-    try:
-        q2 = query.view(tokens, qw)
-    except RuntimeError as e:
-        raise ValueError(f"rotary_embedding: query rows must be [heads*head_size] ({e})") from None
-    if q2.stride(1) != 1:
-        raise ValueError("rotary_embedding: query rows must be contiguous")
-    num_heads = qw // head_size
+    q_stride, num_heads = _token_rows(query, tokens, head_size, "rotary_embedding: query")
     k_stride, num_kv = 0, 0
     if key is not None:
-        kw = key.numel() // tokens
-        if kw % head_size:
-            raise ValueError("rotary_embedding: key width is not a multiple of head_size")
-        try:
-            k2 = key.view(tokens, kw)
-        except RuntimeError as e:
-            raise ValueError(f"rotary_embedding: key rows must be [heads*head_size] ({e})") from None
-        if k2.stride(1) != 1:
-            raise ValueError("rotary_embedding: key rows must be contiguous")
-        k_stride, num_kv = k2.stride(0), kw // head_size
-    _native.call("fk_rotary_embedding", _ptr(positions), _ptr(query), q2.stride(0), _ptr(key),
+        k_stride, num_kv = _token_rows(key, tokens, head_size, "rotary_embedding: key")
+    _native.call("fk_rotary_embedding", _ptr(positions), _ptr(query), q_stride, _ptr(key),
                  k_stride, _ptr(cos_sin_cache), _tag(cos_sin_cache, "rotary cache"),
                  cos_sin_cache.shape[0], tokens, num_heads, num_kv, head_size,
                  cos_sin_cache.shape[1], int(bool(is_neox)), _tag(query, "rotary_embedding"),
@@ -248,6 +238,11 @@ def store_kvcache_hnd(key: torch.Tensor, value: torch.Tensor, k_cache: torch.Ten
 def _token_rows(t: torch.Tensor, tokens: int, head_size: int, what: str) -> tuple[int, int]:
     """(row_stride, heads) of a [tokens, heads*head_size] (or [tokens, heads, head_size])
     view whose rows are contiguous."""
+    if t.dim() == 2:
+        n, w = t.shape
+        s0, s1 = t.stride()
+        if n == tokens and s1 == 1 and w > 0 and w % head_size == 0:
+            return (s0 if n > 1 else w), w // head_size
     w = t.numel() // tokens
     if w % head_size:
         raise ValueError(f"{what}: width {w} is not a multiple of head_size {head_size}")
@@ -274,24 +269,28 @@ def qk_norm_rope_store(positions: torch.Tensor, query: torch.Tensor, key: torch.
     if positions.dtype != torch.int64 or not positions.is_contiguous():
         raise TypeError("qk_norm_rope_store: positions must be contiguous int64")
     tokens = positions.numel()
-    for t, nm in ((key, "key"), (value, "value"), (k_cache, "k_cache"), (v_cache, "v_cache")):
-        if t.dtype != query.dtype:
-            raise TypeError(f"qk_norm_rope_store: {nm} dtype must equal the query dtype")
+    dtype = query.dtype
+    if not (key.dtype == value.dtype == k_cache.dtype == v_cache.dtype == dtype):
+        raise TypeError("qk_norm_rope_store: the key, value, k_cache and v_cache dtypes must "
+                        "equal the query dtype")
+    cs_dtype = cos_sin_cache.dtype
     if cos_sin_cache.dim() != 2 or not cos_sin_cache.is_contiguous() or \
-            cos_sin_cache.dtype not in (torch.float32, query.dtype):
+            (cs_dtype != torch.float32 and cs_dtype != dtype):
         raise ValueError("qk_norm_rope_store: cos_sin_cache must be contiguous float32 or "
                          "query-dtype [max_pos, rot_dim]")
     if (q_weight is None) != (k_weight is None):
         raise ValueError("qk_norm_rope_store: pass both q_weight and k_weight, or neither")
-    for w, nm in ((q_weight, "q_weight"), (k_weight, "k_weight")):
-        if w is not None and (w.dtype != query.dtype or w.numel() != head_size or
-                              not w.is_contiguous()):
-            raise ValueError(f"qk_norm_rope_store: {nm} must be contiguous [head_size] of the "
-                             "query dtype")
-    if slot_mapping.dtype not in (torch.int32, torch.int64) or not slot_mapping.is_contiguous() \
-            or slot_mapping.numel() < tokens:
+    if q_weight is not None:
+        for w, nm in ((q_weight, "q_weight"), (k_weight, "k_weight")):
+            if w.dtype != dtype or w.numel() != head_size or not w.is_contiguous():
+                raise ValueError(f"qk_norm_rope_store: {nm} must be contiguous [head_size] of "
+                                 "the query dtype")
+    slot_i64 = slot_mapping.dtype == torch.int64
+    if not (slot_i64 or slot_mapping.dtype == torch.int32) or \
+            not slot_mapping.is_contiguous() or slot_mapping.numel() < tokens:
         raise TypeError("qk_norm_rope_store: slot_mapping must be contiguous int32/int64 [T]")
-    if k_cache.dim() != 4 or v_cache.shape != k_cache.shape or k_cache.shape[3] != head_size \
+    cache = k_cache.shape
+    if len(cache) != 4 or v_cache.shape != cache or cache[3] != head_size \
             or not (k_cache.is_contiguous() and v_cache.is_contiguous()):
         raise ValueError("qk_norm_rope_store: caches must be contiguous [blocks, bs, Hk, D]")
     _same_device(positions, query, key, value, k_cache, v_cache, slot_mapping, cos_sin_cache)
@@ -300,15 +299,15 @@ def qk_norm_rope_store(positions: torch.Tensor, query: torch.Tensor, key: torch.
     qs, hq = _token_rows(query, tokens, head_size, "qk_norm_rope_store query")
     ks, hk = _token_rows(key, tokens, head_size, "qk_norm_rope_store key")
     vs, hv = _token_rows(value, tokens, head_size, "qk_norm_rope_store value")
-    if hv != hk or k_cache.shape[2] != hk:
+    if hv != hk or cache[2] != hk:
         raise ValueError("qk_norm_rope_store: key, value and caches must have the same kv heads")
-    _native.call("fk_qk_norm_rope_store", _ptr(positions), _ptr(query), qs, _ptr(key), ks,
-                 _ptr(value), vs, _ptr(q_weight), _ptr(k_weight), float(eps),
-                 _ptr(cos_sin_cache), _tag(cos_sin_cache, "rotary cache"),
-                 cos_sin_cache.shape[0], cos_sin_cache.shape[1], int(bool(is_neox)),
-                 _ptr(k_cache), _ptr(v_cache), _ptr(slot_mapping),
-                 int(slot_mapping.dtype == torch.int64), k_cache.shape[0] * k_cache.shape[1],
-                 tokens, hq, hk, head_size, _tag(query, "qk_norm_rope_store"), _stream(query))
+    max_pos, rot_dim = cos_sin_cache.shape
+    _native.call("fk_qk_norm_rope_store", positions.data_ptr(), query.data_ptr(), qs,
+                 key.data_ptr(), ks, value.data_ptr(), vs, _ptr(q_weight), _ptr(k_weight),
+                 float(eps), cos_sin_cache.data_ptr(), _tag(cos_sin_cache, "rotary cache"), max_pos, rot_dim,
+                 1 if is_neox else 0, k_cache.data_ptr(), v_cache.data_ptr(),
+                 slot_mapping.data_ptr(), 1 if slot_i64 else 0, cache[0] * cache[1], tokens, hq,
+                 hk, head_size, _tag(query, "qk_norm_rope_store"), _stream(query))
 
 
 # ---------------------------------------------------------------------------
@@ -331,16 +330,19 @@ def paged_decode_plan(batch: int, num_heads: int, num_kv_heads: int, head_size: 
 
 def _check_decode(out, q, k_cache, v_cache, block_table, cache_seqlens, k_scale, v_scale,
                   window_left=-1, sinks=None):
-    if q.dim() != 3 or q.dtype != torch.bfloat16 or q.stride(2) != 1 or q.stride(1) != q.shape[2]:
+    shape = q.shape
+    if len(shape) != 3 or q.dtype != torch.bfloat16 or q.stride()[1:] != (shape[2], 1):
         raise ValueError("paged_decode: q must be bf16 [B, Hq, D] with contiguous heads")
-    b, hq, d = q.shape
-    if out.shape != q.shape or out.dtype != q.dtype or out.stride(2) != 1 or out.stride(1) != d:
+    b, hq, d = shape
+    if out.shape != shape or out.dtype != torch.bfloat16 or out.stride()[1:] != (d, 1):
         raise ValueError("paged_decode: out must be bf16 [B, Hq, D] with contiguous heads")
-    if k_cache.dim() != 4 or v_cache.shape != k_cache.shape or k_cache.shape[3] != d:
+    cache = k_cache.shape
+    if len(cache) != 4 or v_cache.shape != cache or cache[3] != d:
         raise ValueError("paged_decode: caches must be [num_blocks, block_size, Hk, D]")
     if not (k_cache.is_contiguous() and v_cache.is_contiguous()):
         raise ValueError("paged_decode: caches must be contiguous")
-    if k_cache.dtype != v_cache.dtype or k_cache.dtype not in (torch.bfloat16, _FP8):
+    kv = k_cache.dtype
+    if v_cache.dtype != kv or (kv != torch.bfloat16 and kv != _FP8):
         raise TypeError("paged_decode: caches must both be bf16 or float8_e4m3fn")
     if block_table.dtype != torch.int32 or block_table.dim() != 2 or block_table.stride(1) != 1:
         raise TypeError("paged_decode: block_table must be int32 [B, max_blocks], rows contiguous")
@@ -349,11 +351,11 @@ def _check_decode(out, q, k_cache, v_cache, block_table, cache_seqlens, k_scale,
     if cache_seqlens.dtype != torch.int32 or not cache_seqlens.is_contiguous() or \
             cache_seqlens.numel() < b:
         raise TypeError("paged_decode: cache_seqlens must be contiguous int32 [B]")
-    hk = k_cache.shape[2]
-    for s, nm in ((k_scale, "k_scale"), (v_scale, "v_scale")):
-        if s is not None and (s.dtype != torch.float32 or s.numel() != hk or
-                              not s.is_contiguous()):
-            raise ValueError(f"paged_decode: {nm} must be float32 [num_kv_heads]")
+    if k_scale is not None or v_scale is not None:
+        for s, nm in ((k_scale, "k_scale"), (v_scale, "v_scale")):
+            if s is not None and (s.dtype != torch.float32 or s.numel() != cache[2] or
+                                  not s.is_contiguous()):
+                raise ValueError(f"paged_decode: {nm} must be float32 [num_kv_heads]")
     if int(window_left) < -1:
         raise ValueError("paged_decode: window_left must be -1 (no window) or >= 0")
     if sinks is not None:
@@ -379,12 +381,12 @@ def paged_decode(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor,
     if b == 0:
         return
     nb, bs, hk, _ = k_cache.shape
-    ws_bytes = workspace.numel() * workspace.element_size() if workspace is not None else 0
-    _native.call("fk_paged_decode", _ptr(out), out.stride(0), _ptr(q), q.stride(0),
-                 _ptr(k_cache), _ptr(v_cache),
+    ws_bytes = workspace.nbytes if workspace is not None else 0
+    _native.call("fk_paged_decode", out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0),
+                 k_cache.data_ptr(), v_cache.data_ptr(),
                  _native.FK_DTYPE_FP8_E4M3FN if k_cache.dtype == _FP8 else _native.FK_DTYPE_BF16,
-                 _ptr(k_scale), _ptr(v_scale), _ptr(block_table), block_table.stride(0),
-                 _ptr(cache_seqlens), b, hq, hk, d, bs, nb, float(softmax_scale),
+                 _ptr(k_scale), _ptr(v_scale), block_table.data_ptr(), block_table.stride(0),
+                 cache_seqlens.data_ptr(), b, hq, hk, d, bs, nb, float(softmax_scale),
                  int(window_left), _ptr(sinks), part_tokens, max_parts, _ptr(workspace),
                  ws_bytes, _stream(q))
 
