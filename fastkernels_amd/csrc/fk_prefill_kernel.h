@@ -279,17 +279,23 @@ struct Stage {
 // other stage buffer, which would serialise the double buffer.  The kernel
 // orders it explicitly instead (s_waitcnt vmcnt(0), then a barrier, before the
 // buffer is read).  M0 carries the LDS address: an input operand bound to M0, so
-// the compiler writes it (and knows it changed) with no save and restore; the
-// s_nop is the wait state between that write and the load that reads M0.
+// the compiler writes it (and knows it changed) with no save and restore.  The
+// compiler cannot insert wait states inside the asm, and a VMEM instruction needs
+// five between a VALU write of its base's SGPRs and itself (a v_readlane that
+// reloads a spilled SGPR came four before the load in the paged kernels at heads
+// of 72 and 80).  So the asm copies the base with a scalar move, which hardware
+// interlocks cover on both sides, and which is also the one wait state between
+// the write of M0 and the load (five s_nop states instead cost 1 to 2%).
 // The address is a wave-uniform 64-bit base in SGPRs and a per-lane 32-bit byte
 // offset (the load's saddr form): lane l reads base + off.  A tile's base
 // changes from stage to stage and the lanes' offsets do not, so a stage's
 // loads take no 64-bit address arithmetic per lane.
 __device__ __forceinline__ void lds_dma16_s(const uint8_t* base, uint32_t off, uint32_t lds_addr) {
+  const uint8_t* b;
   asm volatile(
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %0, %1"
-      :
+      "s_mov_b64 %0, %2\n\t"
+      "global_load_lds_dwordx4 %1, %0"
+      : "=&s"(b)
       : "v"(off), "s"(base), "{m0}"(lds_addr)
       : "memory");
 }
