@@ -194,21 +194,24 @@ constexpr int kPrefillWaves = 4;               // waves per work-group
 constexpr int kStageKeys = FK_PREFILL_STAGE;
 constexpr int kStageTiles = kStageKeys / kTile;
 
-__device__ __forceinline__ int64_t prefill_page(const PrefillParams& P,
-                                                const int32_t* __restrict__ bt_row, int tok) {
-  const int idx = tok >> P.block_size_log2;
-  if (idx >= P.bt_row_stride) return -1;
-  const int64_t page = bt_row[idx];
-  return (page >= 0 && page < P.num_blocks) ? page : -1;
-}
-
 // The last block-table entry a wave looked up (wave-uniform), with the K and V
 // rows of its page's first slot (the kv head's row of the caches): a page spans
 // block_size / 32 stages, so most lookups reuse it instead of waiting for a
 // scalar load, and a tile's source address is that row plus a 32-bit offset.
+// Everything but the addresses is 32-bit (the host bounds a page's bytes below
+// 2^32): at 16-token pages every stage looks up two pages, and in 64-bit steps
+// their scalar instructions held up every stage.  Same box, A/B in alternating
+// processes, us, 64-bit -> 32-bit: 1x2048 54.5 -> 46.7, 5 ragged chunks 322.6 ->
+// 285.4, 16x512 70.7 -> 66, 4x512 over 4096 170.7 -> 151.3 (256-token pages 144.7
+// -> 140.5, fp8 205.5 -> 174.7), 13 ragged fp8 prompts 132 -> 117.3, 1x2048 at 16 /
+// 2 / 256 61 -> 57.7, at 20 / 20 / 64 40.4 -> 35.5, 4x512 over 4096 at 64 / 8 / 64
+// 254.5 -> 213.2.
 struct PageCache {
+  int row_entries = 0;           // entries of the table row
+  uint32_t num_blocks = 0;
+  uint32_t k_bytes = 0, v_bytes = 0;  // a page's bytes
   int idx = -1;
-  int64_t page = -1;             // the block-table entry (-1: masked; page 0 is read)
+  int page = -1;                 // the block-table entry (-1: masked; page 0 is read)
   const uint8_t* kb = nullptr;   // K row of the page's slot 0, kv head h
   const uint8_t* vb = nullptr;   // V row of the page's slot 0, kv head h
 };
@@ -220,12 +223,12 @@ __device__ __forceinline__ void page_lookup(const PrefillParams& P,
                                             const uint8_t* kh, const uint8_t* vh, PageCache& pc) {
   const int idx = tok >> P.block_size_log2;
   if (idx != pc.idx) {
-    const int64_t page = prefill_page(P, bt_row, tok);
-    const int64_t slot0 = (page < 0 ? 0 : page) << P.block_size_log2;
+    const int entry = idx < pc.row_entries ? bt_row[idx] : -1;
+    const uint32_t pg = static_cast<uint32_t>(entry) < pc.num_blocks ? entry : 0;
     pc.idx = idx;
-    pc.page = page;
-    pc.kb = kh + slot0 * P.k_row_bytes;
-    pc.vb = vh + slot0 * P.v_row_bytes;
+    pc.page = static_cast<uint32_t>(entry) < pc.num_blocks ? entry : -1;
+    pc.kb = kh + static_cast<uint64_t>(pg) * pc.k_bytes;
+    pc.vb = vh + static_cast<uint64_t>(pg) * pc.v_bytes;
   }
 }
 
@@ -635,6 +638,12 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
   };
 
   PageCache pc;
+  if constexpr (kPaged) {
+    pc.row_entries = static_cast<int>(min(P.bt_row_stride, int64_t(INT_MAX)));
+    pc.num_blocks = static_cast<uint32_t>(min(P.num_blocks, int64_t(INT_MAX)));
+    pc.k_bytes = static_cast<uint32_t>(P.k_row_bytes << P.block_size_log2);
+    pc.v_bytes = static_cast<uint32_t>(P.v_row_bytes << P.block_size_log2);
+  }
   // One query block of the work-group, start to finish: this half streams stages
   // [st_lo, st_hi) of it (st0: the block's first stage) and every wave passes
   // nsteps step barriers; with the key split the halves then merge (unless solo:
