@@ -550,7 +550,7 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
   const int32_t* bt_row = kPaged ? block_tables + static_cast<int64_t>(b) * P.bt_row_stride
                                  : nullptr;
   // Dense keys: rows past the sequence's last key would run off the tensor.
-  const int64_t row_cap = kPaged ? INT64_MAX : static_cast<int64_t>(k_start) + max(k_len, 1) - 1;
+  const int last_row = max(k_len, 1) - 1;  // from row k_start
   // fp8 dequant scales of kv head h (1 for bf16 pages or no scale tensor), one per
   // head: every e4m3fn value is a bf16 value, so K and V enter the MFMAs exactly
   // and K's scale joins the softmax scale, V's the division by the row sum (no
@@ -1038,6 +1038,9 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
   // Row 0 of the caches (paged) or of the tensors (dense) at kv head h.
   const uint8_t* const kh = P.k_cache + k_head_off;
   const uint8_t* const vh = P.v_cache + v_head_off;
+  // Dense keys: the sequence's first rows.
+  const uint8_t* const kd = kPaged ? kh : kh + static_cast<int64_t>(k_start) * P.k_row_bytes;
+  const uint8_t* const vd = kPaged ? vh : vh + static_cast<int64_t>(k_start) * P.v_row_bytes;
   // Slot -> (K or V, row, logical chunk) of load i for this lane.
   auto slot_of = [&](int i, int& which, int& row, int& q) {
     const int pos = 64 * (kPrefillWaves * i + wave) + lane;
@@ -1073,10 +1076,10 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
     const uint32_t buf_addr = stage_addr(st);  // wave-uniform (the buffer is the half's)
     // First K and V rows of the stage's tiles, wave-uniform: paged, the cached
     // page's slot-0 rows plus the slot's 32-bit offset in the page (the host
-    // bounds a page's bytes below 2^32); dense, row k_start + token.
+    // bounds a page's bytes below 2^32); dense, row token of the sequence.
     const uint8_t* kt[kStageTiles];
     const uint8_t* vt[kStageTiles];
-    int64_t row0[kStageTiles];  // dense keys: the tiles' first rows
+    int room[kStageTiles];  // dense keys: rows after the tile's first up to the last one
     bool all_ok = true;
 #pragma unroll
     for (int tt = 0; tt < kStageTiles; ++tt) {
@@ -1087,11 +1090,15 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
         const uint32_t slot = static_cast<uint32_t>(tok) & slot_mask;
         kt[tt] = pc.kb + slot * static_cast<uint32_t>(P.k_row_bytes);
         vt[tt] = pc.vb + slot * static_cast<uint32_t>(P.v_row_bytes);
-        row0[tt] = 0;
+        room[tt] = 15;
       } else {
-        row0[tt] = min(static_cast<int64_t>(k_start) + tok, row_cap);
-        kt[tt] = kh + row0[tt] * P.k_row_bytes;
-        vt[tt] = vh + row0[tt] * P.v_row_bytes;
+        // (32-bit row and row size, as for pages: the host bounds 16 rows below 2^32.
+        // Same box, us, against 64-bit ones: 1x3000 at 16 heads of 80, not causal, 73.3
+        // -> 68.7, of 72 111 -> 104, of 256 140 -> 134.5, MLA chunks 202 -> 197.5.)
+        const int row = min(tok, last_row);
+        kt[tt] = kd + static_cast<uint64_t>(row) * static_cast<uint32_t>(P.k_row_bytes);
+        vt[tt] = vd + static_cast<uint64_t>(row) * static_cast<uint32_t>(P.v_row_bytes);
+        room[tt] = last_row - row;
       }
     }
     if (!all_ok) ok_until = min(ok_until, st);
@@ -1101,14 +1108,14 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
       const int which = pos0 >= S::kNK;                   // 0: K, 1: V
       const int tt = which ? ((pos0 - S::kNK) / S::kVChunks) >> 4 : (pos0 / S::kKChunks) >> 4;
       const uint8_t* base = which ? vt[0] : kt[0];
-      int64_t first = row0[0];
+      int rm = room[0];
 #pragma unroll
       for (int u = 1; u < kStageTiles; ++u)
         if (tt == u) {
           base = which ? vt[u] : kt[u];
-          first = row0[u];
+          rm = room[u];
         }
-      if (kPaged || row_cap - first >= 15) {
+      if (kPaged || rm >= 15) {
         // (padded rows: the padding chunks are not loaded)
         if ((S::kKReal == S::kKChunks && S::kVReal == S::kVChunks) || lane_ld[i])
           lds_dma16_s(base, lane_off[i], buf_addr + 16 * pos0);
@@ -1120,7 +1127,7 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
         // encoder, 16 heads of 80, 219 -> 184.5 us, 1x3000 99.5 -> 72.7).
         int wh, row, q;
         slot_of(i, wh, row, q);
-        const int past = max(0, (row & 15) - static_cast<int>(row_cap - first));
+        const int past = max(0, (row & 15) - rm);
         const uint32_t rb = static_cast<uint32_t>(which ? P.v_row_bytes : P.k_row_bytes);
         if (lane_ld[i])
           lds_dma16_s(base, lane_off[i] - static_cast<uint32_t>(past) * rb, buf_addr + 16 * pos0);
