@@ -71,8 +71,14 @@ PrefillShape prefill_shape(bool paged, bool fp8, int64_t batch, int64_t max_seql
   // work-groups, instead of one 8-wave key-split work-group per block, for
   // chunks over cached keys (blocks not paired) and, at head sizes up to 64 with
   // bf16 pages, for causal pairs.  xs = floor(2 CUs / work-groups) when that is
-  // at least 2 and fills 7/8 of the two-per-CU slots, else the ceiling (at most
-  // kMaxKeyParts), and only while a part keeps at least 20 stages of 32 keys (40
+  // at least 2 and fills 7/8 of the two-per-CU slots; else the parts run in two
+  // rounds of the slots, and xs = floor(4 CUs / work-groups), the most that two
+  // rounds hold (the ceiling of one round's, taken before, ran as many rounds of
+  // longer parts; same box, us, whole call: Qwen3-8B heads 1x800 over 8192 168 ->
+  // 126, 1x1100 over 8192 244 -> 189, over 16000 on fp8 pages 568 -> 403, 2x600 over
+  // 6000 171 -> 135, MLA 877 and 1200 over 2669 and 3300 194.5 -> 167.6; where the
+  // quotients agree nothing changes).  At most kMaxKeyParts, and only while a part
+  // keeps at least 20 stages of 32 keys (40
   // above head size 64: a dense 2048-token non-causal prompt at 16 / 16 / 80
   // heads, 2 parts of 32 stages, went 48.8 -> 52.9).
   // Measured on MI355X (whole call, µs, key split -> this; same box, A/B in
@@ -92,12 +98,16 @@ PrefillShape prefill_shape(bool paged, bool fp8, int64_t batch, int64_t max_seql
       (!may_pair || (!fp8 && std::max(head_size, head_size_v) <= 64))) {
     const int64_t slots = 2 * ncu;
     int64_t xs = slots / wgs;
-    if (xs < 2 || 8 * wgs * xs < 7 * slots) xs = (slots + wgs - 1) / wgs;
+    const bool one_round = xs >= 2 && 8 * wgs * xs >= 7 * slots;
+    if (!one_round) xs = 2 * slots / wgs;
     xs = std::min<int64_t>(xs, kMaxKeyParts);
     const double stages = static_cast<double>(std::max(max_seqlen_k, max_seqlen_q) +
                                               (may_pair ? wg_tokens : 0)) /
                           kStageKeys;  // the heaviest work-group's stages (a pair's)
     const double min_stages = std::max(head_size, head_size_v) <= 64 ? 20.0 : 40.0;
+    // (Keys too few for the parts of two rounds: the fewest that leave no slot idle.)
+    if (!one_round && stages < min_stages * xs)
+      xs = std::min<int64_t>((slots + wgs - 1) / wgs, kMaxKeyParts);
     if (xs >= 2 && stages >= min_stages * xs && sh.qblocks * xs <= 65535) {
       sh.ks = 1;
       sh.xs = static_cast<int>(xs);
