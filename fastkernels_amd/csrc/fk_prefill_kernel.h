@@ -151,7 +151,7 @@ constexpr int kQTokens = 16 * kColBlocks;      // query tokens per wave at head 
 // 192 / 128 takes two (246 registers): each K / V byte read from LDS then serves
 // 32 queries, and a work-group 128 instead of 64.  Same box, us: 877 and 1200 new
 // tokens over 2669 and 3300 cached ones, 16 heads (both calls and the merge) 249
-// -> 206; 300 .. 2000 over 500 .. 1500 178 -> 160; 1x256 over 8192 unchanged (64).
+// -> 198; 300 .. 2000 over 500 .. 1500 178 -> 157; 1x256 over 8192 unchanged (64).
 constexpr int col_blocks_for(int D, int DV) { return (D > 192 || DV > 128) ? 1 : kColBlocks; }
 // MFMA extents: the score MFMAs run over D rounded up to 32, P.V over DV rounded
 // up to 16.
@@ -1124,7 +1124,7 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
         // read that row (their 32-bit offset taken back by the rows they are past
         // it; 64-bit row addresses here took 10 to 20 registers more in every dense
         // kernel, at heads of 72 and 80 the third wave per SIMD: ragged vision
-        // encoder, 16 heads of 80, 219 -> 184.5 us, 1x3000 99.5 -> 72.7).
+        // encoder, 16 heads of 80, 219 -> 181 us, 1x3000 99.5 -> 72).
         int wh, row, q;
         slot_of(i, wh, row, q);
         const int past = max(0, (row & 15) - rm);
