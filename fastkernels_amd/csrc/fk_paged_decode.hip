@@ -1351,6 +1351,49 @@ int solo_shares(int64_t batch, int vheads, int head_size, int window_left) {
   return tiles <= most * kSoloShort ? most : 0;
 }
 
+// How a launch is divided: virtual heads (waves) per work-group, as the kernels are
+// instantiated, waves per virtual head (DecodeParams::split), and the LDS its waves
+// merge through.  waves * shares is at most kMaxWavesPerGroup: the partition kernel
+// is bounded to that many waves.
+struct DecodeShape {
+  bool whole;  // whole windows (DecodeParams::solo)
+  int waves;
+  int shares;
+  size_t lds;
+};
+DecodeShape decode_shape(int64_t batch, int vheads, int head_size, int window_left,
+                         int64_t part_tokens, int64_t max_parts) {
+  const bool balanced = part_tokens == 0;
+  // Rounded up to a power of two: 3 heads run as 4 waves with one idle.
+  int p2 = 1;
+  while (p2 < waves_per_group(vheads)) p2 *= 2;
+  DecodeShape sh = {false, p2, 1, 0};
+  if (const int s = balanced ? solo_shares(batch, vheads, head_size, window_left) : 0) {
+    // Work-groups of 8 waves or fewer whose states fit in 64 KB of LDS.
+    sh.whole = true;
+    sh.shares = s;
+    sh.waves = 1;
+    while (2 * sh.waves * s <= kMaxWavesPerGroup && 2 * sh.waves <= vheads &&
+           solo_lds(2 * sh.waves, s, head_size) <= kSoloLds)
+      sh.waves *= 2;
+    sh.lds = solo_lds(sh.waves, s, head_size);
+    return sh;
+  }
+  if (balanced) return sh;
+  // Fixed partitions: while the grid holds fewer work-groups than CUs (few partitions
+  // of a small batch), fewer virtual heads per work-group and more work-groups.
+  while (sh.waves > 1 &&
+         max_parts * batch * ((vheads + sh.waves - 1) / sh.waves) < num_cus())
+    sh.waves /= 2;
+  // Those that would run one wave per SIMD (or fewer) split each partition over two
+  // waves of the work-group.
+  if (sh.waves <= 4 && max_parts * batch * vheads < 2LL * 4 * num_cus()) {
+    sh.shares = 2;
+    sh.lds = solo_lds(sh.waves, 2, head_size);
+  }
+  return sh;
+}
+
 struct Launch {
   DecodeParams P;
   const void* slot_mapping = nullptr;
@@ -1359,7 +1402,7 @@ struct Launch {
   int nh;
   int head_size;
   dim3 grid;
-  size_t part_lds = 0;  // fixed partitions split over two waves: the merge area
+  size_t part_lds = 0;  // partitions in shares: the merge area
 };
 
 int prepare(const char* name, Launch& L, void* out, int64_t out_row_stride, const void* q,
@@ -1435,46 +1478,20 @@ int prepare(const char* name, Launch& L, void* out, int64_t out_row_stride, cons
   L.fp8 = kv_dtype == FK_DTYPE_FP8_E4M3FN;
   L.head_size = head_size;
   const int vh = virtual_heads(num_heads, num_kv_heads);
-  L.nh = waves_per_group(vh);
-  if (!balanced) {
-    // Fixed partitions: while the grid holds fewer work-groups than CUs (few
-    // partitions of a small batch), fewer virtual heads per work-group (a
-    // power of two, as the launches take) and more work-groups.
-    while (L.nh > 1 && static_cast<int64_t>(max_parts) * batch * ((vh + L.nh - 1) / L.nh) <
-                           num_cus()) {
-      int p2 = 1;
-      while (2 * p2 < L.nh) p2 *= 2;
-      L.nh = p2;
-    }
-  }
-  // Fixed partitions that would run one wave per SIMD (or fewer) split each
-  // partition over two waves of the work-group.
-  P.split = 1;
-  P.solo = 0;
-  if (const int s = balanced ? solo_shares(batch, vh, head_size, window_left) : 0) {
+  const DecodeShape sh = decode_shape(batch, vh, head_size, window_left, part_tokens, max_parts);
+  L.nh = sh.waves;
+  L.part_lds = sh.lds;
+  P.split = sh.shares;
+  P.solo = sh.whole ? 1 : 0;
+  if (sh.whole) {
     L.balanced = false;
-    P.solo = 1;
     P.part_tokens = 1 << 30;
     P.max_parts = 1;
-    P.split = s;
-    // Work-groups of 8 waves or fewer whose states fit in 64 KB of LDS.
-    int nh = 1;
-    while (2 * nh * s <= kMaxWavesPerGroup && 2 * nh <= vh &&
-           solo_lds(2 * nh, s, head_size) <= kSoloLds)
-      nh *= 2;
-    L.nh = nh;
-    L.part_lds = solo_lds(nh, s, head_size);
-    L.grid = dim3(1, static_cast<unsigned>((vh + nh - 1) / nh), static_cast<unsigned>(batch));
-    return FK_OK;
-  }
-  if (!balanced && L.nh <= 4 &&
-      static_cast<int64_t>(max_parts) * batch * vh < 2LL * 4 * num_cus()) {
-    P.split = 2;
-    L.part_lds = static_cast<size_t>(L.nh) * (head_size / 16 * 4 * 64 + 2 * 64) * sizeof(float);
   }
   const unsigned hgroups = static_cast<unsigned>((vh + L.nh - 1) / L.nh);
-  L.grid = balanced ? dim3(static_cast<unsigned>(max_parts), hgroups, 1)
-                    : dim3(static_cast<unsigned>(max_parts), hgroups, static_cast<unsigned>(batch));
+  L.grid = L.balanced ? dim3(static_cast<unsigned>(max_parts), hgroups, 1)
+                      : dim3(static_cast<unsigned>(P.max_parts), hgroups,
+                             static_cast<unsigned>(batch));
   return FK_OK;
 }
 
@@ -1622,6 +1639,22 @@ extern "C" int fk_paged_decode_plan(int64_t batch, int num_heads, int num_kv_hea
   }
   *workspace_bytes_out =
       batch > 0 ? workspace_bytes(*part_tokens == 0, batch, num_heads, head_size, *max_parts) : 0;
+  return FK_OK;
+}
+
+extern "C" int fk_paged_decode_shape(int64_t batch, int num_heads, int num_kv_heads,
+                                     int head_size, int window_left, int64_t part_tokens,
+                                     int64_t max_parts, int* waves, int* shares,
+                                     int* whole_windows) {
+  const char* name = "fk_paged_decode_shape";
+  FK_REQUIRE(waves && shares && whole_windows, "%s: null output pointer", name);
+  const int rc = validate(name, batch, num_heads, num_kv_heads, head_size, part_tokens, max_parts);
+  if (rc != FK_OK) return rc;
+  const DecodeShape sh = decode_shape(batch, virtual_heads(num_heads, num_kv_heads), head_size,
+                                      window_left, part_tokens, max_parts);
+  *waves = sh.waves;
+  *shares = sh.shares;
+  *whole_windows = sh.whole ? 1 : 0;
   return FK_OK;
 }
 

@@ -77,7 +77,9 @@ extern "C" {
  * whenever an existing entry point's signature changes; a caller built against this
  * header checks fk_version() / 10000 == FK_VERSION_MAJOR before binding. */
 #define FK_VERSION_MAJOR 2
-#define FK_VERSION_MINOR 1 /* 2.1: fk_prefill_split_plan, fk_paged_prefill_ws, fk_varlen_prefill_ws */
+/* 2.1: fk_prefill_split_plan, fk_paged_prefill_ws, fk_varlen_prefill_ws
+ * 2.2: fk_paged_decode_shape */
+#define FK_VERSION_MINOR 2
 int fk_version(void);
 
 /* Message describing the last failing call on this thread ("" if none). */
@@ -156,6 +158,17 @@ int fk_store_kvcache_hnd(const void* key, int64_t key_row_stride, const void* va
 int fk_paged_decode_plan(int64_t batch, int num_heads, int num_kv_heads, int head_size,
                          int64_t max_seq_len, int num_splits, int64_t* part_tokens,
                          int64_t* max_parts, int64_t* workspace_bytes);
+
+/* How fk_paged_decode launches such a plan (host-only, for tests and profiling):
+ *   waves:         waves per work-group that take a kv head (or a block of 16 of its
+ *                  query heads) each: 1, 2, 4 or 8.
+ *   shares:        waves that divide one such head's tiles and merge in LDS; a
+ *                  work-group has waves * shares <= 8 waves.
+ *   whole_windows: 1 when, under a sliding window, a work-group takes each sequence's
+ *                  whole window (no merge launch). */
+int fk_paged_decode_shape(int64_t batch, int num_heads, int num_kv_heads, int head_size,
+                          int window_left, int64_t part_tokens, int64_t max_parts, int* waves,
+                          int* shares, int* whole_windows);
 
 /* Paged decode attention (one query token per sequence, at position ctx_lens[b] - 1):
  *   out[b,h,:] = softmax(scale * q[b,h,:] . K_b^T) V_b  over tokens [lo_b, ctx_lens[b])

@@ -154,6 +154,33 @@ def test_plan_host_logic(lib):
         _native.plan(-1, 32, 8, 128, 10, 0)
 
 
+def test_decode_work_groups_fit_the_kernel(lib):
+    """A work-group of the partition kernel has waves * shares waves of 64 lanes, bounded to
+    512 threads; waves is one of the counts the kernels are built for and covers the heads
+    (three heads used to run as eight waves in two shares: 1024 threads)."""
+    from fastkernels_amd import _native
+
+    shares_seen = set()
+    for hk in (1, 2, 3, 4, 5, 6, 7, 8, 9, 11, 20):
+        for group in (1, 3, 16, 17, 40):
+            for d in (64, 128, 256):
+                for batch in (1, 3, 17, 60, 100, 300, 5000):
+                    for part, parts, window in ((512, 1, -1), (512, 4, -1), (512, 16, 100),
+                                                (0, 256, -1), (0, 256, 0), (0, 256, 127),
+                                                (0, 256, 1023), (0, 256, 5000)):
+                        waves, shares, whole = _native.decode_shape(batch, hk * group, hk, d,
+                                                                    window, part, parts)
+                        what = (batch, hk * group, hk, d, window, part, parts)
+                        assert waves in (1, 2, 4, 8) and shares in (1, 2, 4, 8), what
+                        assert waves * shares <= 8, what
+                        assert whole <= (part == 0 and window >= 0), what
+                        assert shares == 1 or whole or part > 0, what
+                        shares_seen.add((whole, shares))
+    assert shares_seen == {(False, 1), (False, 2), (True, 1), (True, 2), (True, 4), (True, 8)}
+    # The shape that made the illegal work-group: 3 kv heads, 100 sequences, 4 partitions.
+    assert _native.decode_shape(100, 9, 3, 64, -1, 512, 4) == (4, 2, False)
+
+
 def test_argument_errors_return_before_launch(lib):
     from fastkernels_amd import _native as N
 

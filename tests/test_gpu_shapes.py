@@ -50,6 +50,17 @@ def test_decode_shapes_bf16(cuda, label, hq, hk, d, num_splits):
     assert_close(got, ref, BF16_TOL, BF16_TOL, f"{label} splits={num_splits}")
 
 
+@pytest.mark.parametrize("batch,splits", [(100, 4), (100, 0), (200, 4), (3, 4)])
+def test_decode_three_kv_heads(cuda, batch, splits):
+    """Three kv heads run as four waves, one idle: fixed partitions in two shares (100
+    sequences), whole (200) and over smaller work-groups (3), and the balanced schedule."""
+    _flush(f"decode 9/3/64 batch {batch} splits={splits}")
+    case = workloads.c3_decode(cuda, batch=batch, num_heads=9, kv_heads=3, head_dim=64,
+                               block_size=16, pool_blocks=8192, ctx_lo=0, ctx_hi=500, seed=batch)
+    assert_close(f32(run_decode(case, splits)), oracle_decode(case), BF16_TOL, BF16_TOL,
+                 f"9/3/64 batch {batch}")
+
+
 @pytest.mark.parametrize("label,hq,hk,d", [SHAPES[0], SHAPES[2], SHAPES[4]])
 def test_decode_shapes_fp8(cuda, label, hq, hk, d):
     _flush(f"decode shape fp8 {label}")
