@@ -57,6 +57,8 @@
 //   FK_DECODE_LDS_STAGE  bf16, head size 128, plain decode: K/V tiles go from
 //     HBM straight to LDS (global_load_lds_dwordx4) through a two-stage ring
 //     per wave, so the next tile's loads are in flight while a tile is used.
+#include <limits.h>
+
 #include "fk_attn_tile.h"
 
 namespace fk {
@@ -166,6 +168,11 @@ __device__ __forceinline__ int64_t page_of(const DecodeParams& P, const int32_t*
 // First visible key of a sequence of ctx tokens under the sliding window.
 __device__ __forceinline__ int key_lo(const DecodeParams& P, int ctx) {
   return P.window_left >= 0 ? max(0, ctx - 1 - P.window_left) : 0;
+}
+
+// Partitions that hold tokens of a sequence of ctx > 0 tokens.
+__device__ __forceinline__ int parts_of(const DecodeParams& P, int ctx) {
+  return min((ctx - 1) / P.part_tokens + 1, P.max_parts);
 }
 
 // Sink logit of query head hq in the kernel's log2 units (scale * q . k
@@ -787,7 +794,9 @@ __attribute__((amdgpu_waves_per_eu(FK_DECODE_WAVES_PER_EU))) void paged_decode_p
   const int p = blockIdx.x;
   const int b = blockIdx.z;
   const int ctx = ctx_lens[b];
-  const int tok_begin = p * P.part_tokens;
+  // (int32 contexts and part_tokens up to 2^30: no product or sum here may wrap.)
+  const int tok_begin =
+      static_cast<int>(min(static_cast<int64_t>(p) * P.part_tokens, static_cast<int64_t>(INT_MAX)));
   // Wave index made provably uniform so that page lookups are scalar loads.
   const int wave_id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wave = wave_id & (NH - 1);  // the virtual-head slot
@@ -801,8 +810,9 @@ __attribute__((amdgpu_waves_per_eu(FK_DECODE_WAVES_PER_EU))) void paged_decode_p
     // The launch has max_parts partitions; the last one runs on to the context
     // end, so a context longer than the plan's max_seq_len bound (a graph
     // replayed after contexts grew) is still attended whole.
-    const int tok_end = p == P.max_parts - 1 ? ctx : min(ctx, tok_begin + P.part_tokens);
-    const int nparts = min((ctx + P.part_tokens - 1) / P.part_tokens, P.max_parts);
+    const bool last = p == P.max_parts - 1 || ctx - tok_begin <= P.part_tokens;
+    const int tok_end = last ? ctx : tok_begin + P.part_tokens;
+    const int nparts = parts_of(P, ctx);
     const int r = lane & 15;
     const int g = lane >> 4;
     // Under a sliding window a partition starts no earlier than the tile of the
@@ -1203,7 +1213,7 @@ __global__ __launch_bounds__(kWaves * 64) void paged_decode_partition_reduce_ker
       zero_row<D>(out_b + static_cast<int64_t>(hq0 + wave) * D, lane);
     return;
   }
-  const int nparts = min((ctx + P.part_tokens - 1) / P.part_tokens, P.max_parts);
+  const int nparts = parts_of(P, ctx);
   if (nparts <= 1) return;  // written by the partition kernel
   const int64_t first = static_cast<int64_t>(b) * P.max_parts * P.num_heads;
   merge_group<D, kRows, kWaves>(P, out_b, hq0, first, first, P.num_heads, nparts, wave, lane);

@@ -77,3 +77,30 @@ def test_whole_windows_match_partitions(cuda, batch, hq, hk, d, window, fp8):
     assert bool(torch.equal(want.view(torch.int16), got.view(torch.int16)))
     assert bool(torch.equal(kc.view(torch.uint8), case.k_cache.view(torch.uint8)))
     assert bool(torch.equal(vc.view(torch.uint8), case.v_cache.view(torch.uint8)))
+
+
+@pytest.mark.parametrize("splits", [0, 1, 2])
+def test_window_of_a_context_past_2_30(cuda, splits):
+    """int32 lengths reach past 2^30 tokens, where a partition count formed as (ctx +
+    part - 1) / part wraps.  Pages of 2^16 tokens, all but the last two unmapped; the
+    window's 101 keys against float64 over them."""
+    print(f"window of a context past 2^30, splits={splits}", flush=True)
+    page, hq, hk, d, window, ctx = 1 << 16, 2, 1, 64, 100, (1 << 30) + 37
+    g = torch.Generator(device=cuda).manual_seed(3)
+    q = torch.randn(1, hq, d, generator=g, device=cuda).to(torch.bfloat16)
+    kc, vc = (torch.randn(2, page, hk, d, generator=g, device=cuda).to(torch.bfloat16)
+              for _ in range(2))
+    pages = -(-ctx // page)
+    bt = torch.full((1, pages), -1, dtype=torch.int32, device=cuda)
+    bt[0, -2], bt[0, -1] = 1, 0  # the window starts in the page before the last
+    part, parts, nbytes = ops.paged_decode_plan(1, hq, hk, d, 1 << 30, splits)
+    ws = torch.zeros(max(1, nbytes), dtype=torch.uint8, device=cuda)
+    out = torch.full_like(q, float("nan"))
+    ops.paged_decode(out, q, kc, vc, bt, torch.tensor([ctx], dtype=torch.int32, device=cuda),
+                     d ** -0.5, part, parts, ws, window_left=window)
+    torch.cuda.synchronize()
+    n = ctx - (pages - 1) * page  # tokens in the last page
+    k = torch.cat([kc[1, page - (window + 1 - n):, 0], kc[0, :n, 0]]).double()
+    v = torch.cat([vc[1, page - (window + 1 - n):, 0], vc[0, :n, 0]]).double()
+    want = torch.softmax(q[0].double() @ k.T * d ** -0.5, -1) @ v
+    torch.testing.assert_close(out[0].double(), want, rtol=1e-2, atol=1e-2)
