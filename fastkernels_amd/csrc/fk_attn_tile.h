@@ -69,6 +69,18 @@ __device__ __forceinline__ uint2 fp8x4_to_bf16x4(uint32_t w) {
       __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.f, true)));
 }
 
+// The same values by way of fp32, four instructions instead of two.  K at head size 128
+// takes it: 64 / 8 / 128 heads, fp8 pages, us, two -> four instructions: 16 x (1333 ..
+// 4000) 28.4 -> 27.2, 4 x (5333 .. 16000) 29.5 -> 28.7, 16 x (5333 .. 16000) 78.9 ->
+// 79.4; at 64 and 256 four cost 5 to 10 % of the long contexts.
+__device__ __forceinline__ uint2 fp8x4_to_bf16x4_by_f32(uint32_t w) {
+  const auto lo = __builtin_amdgcn_cvt_pk_f32_fp8(w, false);
+  const auto hi = __builtin_amdgcn_cvt_pk_f32_fp8(w, true);
+  const bf16x2_t a = {static_cast<__bf16>(lo[0]), static_cast<__bf16>(lo[1])};
+  const bf16x2_t b = {static_cast<__bf16>(hi[0]), static_cast<__bf16>(hi[1])};
+  return make_uint2(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b));
+}
+
 // KV loads (plain cached loads: marking them non-temporal measured slower).
 __device__ __forceinline__ uint4 ld16(const uint8_t* p) { return *reinterpret_cast<const uint4*>(p); }
 __device__ __forceinline__ uint2 ld8(const uint8_t* p) { return *reinterpret_cast<const uint2*>(p); }
@@ -196,7 +208,8 @@ __device__ __forceinline__ void k_chunks_d(const DTile<kFp8, D>& t, uint4 (&kc)[
       const uint4& src = t.k[c >> 1];
       const uint32_t w0 = (c & 1) ? src.z : src.x;
       const uint32_t w1 = (c & 1) ? src.w : src.y;
-      const uint2 lo = fp8x4_to_bf16x4(w0), hi = fp8x4_to_bf16x4(w1);
+      const uint2 lo = D == 128 ? fp8x4_to_bf16x4_by_f32(w0) : fp8x4_to_bf16x4(w0);
+      const uint2 hi = D == 128 ? fp8x4_to_bf16x4_by_f32(w1) : fp8x4_to_bf16x4(w1);
       kc[c] = make_uint4(lo.x, lo.y, hi.x, hi.y);
     }
   }

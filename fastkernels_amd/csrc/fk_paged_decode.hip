@@ -345,6 +345,7 @@ struct WaveState {
   uint8_t* ring;  // kLds: this wave's two LDS stages
   float m_run;  // running max of column r (same in the 4 lanes of a column)
   float l_run;  // this lane's share of the running sum of column r
+  float vsc;    // V's fp8 dequant scale of the kv head (1 for bf16 pages or no scale tensor)
   floatx4_t o[kSl];
 
   // Keys below key_lo (the sliding window's start) are masked; tok_begin is
@@ -408,9 +409,18 @@ struct WaveState {
         qb[c] = __builtin_bit_cast(bf16x8_t, v);
       }
     }
-    // K's fp8 dequant scale (one per kv head) joins the softmax scale; V's is
-    // applied when the rows are written (v_scale_of).
-    const float s2 = (kFp8 && P.k_scale) ? P.scale_log2 * P.k_scale[kvh] : P.scale_log2;
+    // fp8 dequant scales of the kv head: K's multiplies the scores, V's the rows when
+    // they are written.  Both are loaded here and first waited for with tile data in
+    // hand.  (A product of K's scale and the softmax scale is formed before the first
+    // tile's loads are issued and waits there, and V's scale loaded with the rows ends
+    // every segment with its latency.  fp8 pages, kernel with merge, us, both so -> now:
+    // 32 / 8 / 128 heads, one context of 60 8.2 -> 7.9, 16 of 333 .. 1000 15.1 -> 14.0,
+    // 64 of 333 .. 1000 27.4 -> 25.9; 8 / 1 / 128 64 of 333 .. 1000 14.5 -> 13.4.)
+    float ks = 1.f;
+    vsc = 1.f;
+    if (kFp8 && P.k_scale) ks = P.k_scale[kvh];
+    if (kFp8 && P.v_scale) vsc = P.v_scale[kvh];
+    const float s2 = P.scale_log2;
 
     m_run = kNegInf;
     l_run = 0.f;
@@ -499,7 +509,7 @@ struct WaveState {
       const bool full = page >= 0 && tok0 >= key_lo && tok0 + kTile <= tok_end;
       float s[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) s[i] = acc[i] * s2;
+      for (int i = 0; i < 4; ++i) s[i] = kFp8 ? acc[i] * ks * s2 : acc[i] * s2;
       if (!full) {
 #pragma unroll
         for (int i = 0; i < 4; ++i)
@@ -688,15 +698,9 @@ struct WaveState {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the ring is free for the next segment
   }
 
-  // V's fp8 dequant scale of kv head kvh (1 for bf16 pages or no scale tensor).
-  __device__ __forceinline__ static float v_scale_of(const DecodeParams& P, int kvh) {
-    return (kFp8 && P.v_scale) ? P.v_scale[kvh] : 1.f;
-  }
-
   // Normalised output rows of the virtual head for a sequence finished in place.
   __device__ __forceinline__ void write_final(const DecodeParams& P, int b, const VHead& vh,
                                               int r, int g) const {
-    const float vsc = v_scale_of(P, vh.kvh);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int j = 4 * g + i;
@@ -730,7 +734,6 @@ struct WaveState {
   // the virtual head's query heads hq.
   __device__ __forceinline__ void write_partial(const DecodeParams& P, int64_t row0,
                                                 const VHead& vh, int r, int g) const {
-    const float vsc = v_scale_of(P, vh.kvh);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int j = 4 * g + i;
