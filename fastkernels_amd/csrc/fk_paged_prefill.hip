@@ -357,10 +357,11 @@ int prefill_entry(const char* name, bool paged, void* out, int64_t out_row_strid
   FK_REQUIRE(qblocks <= 65535, "%s: max_seqlen_q %lld needs more than 65535 query blocks", name,
              (long long)max_seqlen_q);
   // Longest items first: up to 64 sequences (one per lane of the kernel's ordering).
-  // Items: at most ceil(q_len / block) per sequence.
+  // Items: at most ceil(q_len / block) per sequence, and with a workspace (whose size
+  // total_q was already bounded by) no more than total_q rows hold.
   const int64_t wg_tokens = prefill_wg_tokens(P.gqa, head_size, head_size_v);
   int64_t items = batch * qblocks;
-  if (total_q > 0) items = std::min(items, total_q / wg_tokens + batch);
+  if (workspace != nullptr && total_q > 0) items = std::min(items, total_q / wg_tokens + batch);
   P.lpt = (batch <= 64 && items * sh.xs <= 65535) ? static_cast<int>(batch) : 0;
   const dim3 grid =
       P.lpt ? dim3(static_cast<unsigned>(num_kv_heads * sh.hsplit),

@@ -500,6 +500,15 @@ def _split_workspace(q, paged, kv_dtype, batch, max_seqlen_q, max_seqlen_k, hk, 
     return torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes > 0 else None
 
 
+def _workspace_args(ws, q):
+    """(workspace, bytes) of the _ws entry points.  A launch that does not split takes any
+    workspace of 0 bytes; one that is not NULL lets q's row count bound the grid (64
+    prompts of 16 .. 2000 tokens: 1115 -> 1025 us)."""
+    if ws is not None:
+        return ws.data_ptr(), ws.numel()
+    return (q.data_ptr() if PREFILL_SPLIT else None), 0
+
+
 def paged_prefill(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor,
                   v_cache: torch.Tensor, block_table: torch.Tensor, cu_seqlens_q: torch.Tensor,
                   cu_seqlens_k: torch.Tensor, max_seqlen_q: int, softmax_scale: float,
@@ -549,7 +558,7 @@ def paged_prefill(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor,
                  _ptr(cu_seqlens_q), _ptr(cu_seqlens_k), batch, int(max_seqlen_q),
                  int(max_seqlen_k), q.shape[1], hk, q.shape[2], dv, bs, nb,
                  float(softmax_scale), int(bool(causal)), int(window_left), _ptr(sinks),
-                 q.shape[0], _ptr(ws), 0 if ws is None else ws.numel(), _stream(q))
+                 q.shape[0], *_workspace_args(ws, q), _stream(q))
 
 
 def varlen_prefill(out: torch.Tensor, q: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
@@ -589,7 +598,7 @@ def varlen_prefill(out: torch.Tensor, q: torch.Tensor, key: torch.Tensor, value:
                  _ptr(cu_seqlens_k), batch, int(max_seqlen_q), int(max_seqlen_k), q.shape[1],
                  key.shape[1], q.shape[2], dv, float(softmax_scale), int(bool(causal)),
                  int(window_left), _ptr(sinks), _ptr(lse), 0 if lse is None else lse.stride(0),
-                 q.shape[0], _ptr(ws), 0 if ws is None else ws.numel(), _stream(q))
+                 q.shape[0], *_workspace_args(ws, q), _stream(q))
 
 
 def paged_decode_phases(out, q, k_cache, v_cache, block_table, cache_seqlens, softmax_scale,

@@ -340,9 +340,11 @@ int fk_prefill_split_plan(int paged, int kv_dtype, int64_t batch, int64_t total_
                           int64_t* workspace_bytes);
 
 /* fk_paged_prefill / fk_varlen_prefill with the work-group key split's workspace:
- * workspace NULL runs exactly the entry point without _ws; otherwise
- * workspace_bytes must be at least fk_prefill_split_plan's figure for the same
- * arguments (else FK_ERR_WORKSPACE) and the workspace 16-byte aligned.  Its contents
+ * workspace NULL runs exactly the entry point without _ws (total_q is ignored);
+ * otherwise workspace_bytes must be at least fk_prefill_split_plan's figure for the same
+ * arguments (else FK_ERR_WORKSPACE), the workspace 16-byte aligned, and total_q >=
+ * cu_seqlens_q[batch]: it bounds the work-groups launched, so rows past it may be left
+ * unwritten.  Its contents
  * need no initialisation and are scratch after the call; calls that share a
  * workspace must be ordered (the same stream).  Results match the entry point
  * without _ws to rounding (each part's O is kept in bf16 before the division by its

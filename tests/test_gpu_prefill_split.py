@@ -206,6 +206,38 @@ def test_paged_prefill_ws_entry_point_contract(cuda):
     P._close(split, P._oracle(c), 1e-2, "ws entry point")
 
 
+@pytest.mark.parametrize("total_q", [0, 1, 40])
+def test_prefill_null_workspace_ignores_total_q(cuda, total_q):
+    """Without a workspace total_q says nothing, whatever its value: the same bits as
+    fk_paged_prefill / fk_varlen_prefill, every row written."""
+    _flush(f"prefill NULL workspace, total_q {total_q}")
+    lib = _native.lib()
+    c = P._case(cuda, [200, 3, 90, 300], [700, 3, 400, 300], hq=8, hk=2, bs=16, seed=441)
+    q, batch = c["q"], c["cu_q"].numel() - 1
+    k, v = (torch.randn(1500, 2, 128, device=cuda).to(torch.bfloat16) for _ in range(2))
+
+    def run(entry, *tail):
+        out = torch.full_like(q, float("nan"))
+        head = [ops._ptr(out), out.stride(0), ops._ptr(q), q.stride(0)]
+        shape = [ops._ptr(c["cu_q"]), ops._ptr(c["cu_k"]), batch, c["max_q"], c["max_k"],
+                 q.shape[1], 2, 128, 128]
+        if "paged" in entry:
+            args = head + [ops._ptr(c["kc"]), ops._ptr(c["vc"]), _native.FK_DTYPE_BF16, None,
+                           None, ops._ptr(c["bt"]), c["bt"].stride(0)] + shape + \
+                [16, c["kc"].shape[0], float(c["scale"]), 1, -1, None]
+        else:
+            args = head + [ops._ptr(k), k.stride(0), ops._ptr(v), v.stride(0)] + shape + \
+                [float(c["scale"]), 1, -1, None, None, 0]
+        assert getattr(lib, entry)(*args, *tail, None) == 0
+        torch.cuda.synchronize()
+        return out
+
+    for name in ("fk_paged_prefill", "fk_varlen_prefill"):
+        plain = run(name)
+        assert torch.isfinite(plain).all()
+        assert torch.equal(run(name + "_ws", total_q, None, 0), plain), name
+
+
 def test_prefill_split_plan_sizes():
     """The plan's workspace: parts x rows x heads x (value head size bf16 + 4 fp32),
     rounded up to 256 bytes; zero for launches that fill the GPU and for empty calls."""
