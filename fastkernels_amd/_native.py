@@ -88,6 +88,9 @@ _SIGNATURES = {
                                   c_void_p, c_void_p, c_int64, c_void_p]),
     "fk_prefill_split_plan": (c_int, [c_int, c_int, c_int64, c_int64, c_int64, c_int64, c_int,
                                       c_int, c_int, c_int, c_int, ctypes.POINTER(c_int64)]),
+    "fk_prefill_shape": (c_int, [c_int, c_int, c_int64, c_int64, c_int64, c_int64, c_int, c_int,
+                                 c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p,
+                                 c_void_p]),
     "fk_paged_prefill_ws": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p,
                                     c_int, c_void_p, c_void_p, c_void_p, c_int64, c_void_p,
                                     c_void_p, c_int64, c_int64, c_int64, c_int, c_int, c_int,
@@ -169,6 +172,18 @@ def prefill_split_bytes(paged: bool, kv_dtype: int, batch: int, total_q: int, ma
                                       max_seqlen_k, num_heads, num_kv_heads, head_size,
                                       head_size_v, int(bool(causal)), ctypes.byref(ws)))
     return ws.value
+
+
+def prefill_shape(paged: bool, kv_dtype: int, batch: int, total_q: int, max_seqlen_q: int,
+                  max_seqlen_k: int, num_heads: int, num_kv_heads: int, head_size: int,
+                  head_size_v: int, causal: bool, window_left: int = -1,
+                  with_workspace: bool = True) -> tuple[int, int, int, int]:
+    """fk_prefill_shape: (wg_tokens, key_split, parts, longest_first) of a prefill launch."""
+    out = (c_int * 4)()
+    call("fk_prefill_shape", int(paged), kv_dtype, batch, total_q, max_seqlen_q, max_seqlen_k,
+         num_heads, num_kv_heads, head_size, head_size_v, int(bool(causal)), window_left,
+         int(with_workspace), *(ctypes.byref(out, 4 * i) for i in range(4)))
+    return tuple(out)
 
 
 def plan(batch: int, num_heads: int, num_kv_heads: int, head_size: int, max_seq_len: int,

@@ -37,8 +37,10 @@ int64_t prefill_wg_tokens(int gqa, int head_size, int head_size_v) {
 // Launch shape of a prefill call, from the host-side bounds alone (the plan
 // entry point and the launch agree on it).
 struct PrefillShape {
-  int64_t qblocks;  // query blocks per sequence (grid z before the key parts)
-  int hsplit;       // work-groups per kv head (head groups of up to 4)
+  int64_t wg_tokens;  // query tokens per work-group
+  int64_t qblocks;    // query blocks per sequence (grid z before the key parts)
+  bool may_pair;      // causal pairs of blocks may occur
+  int hsplit;         // work-groups per kv head (head groups of up to 4)
   int ks;           // key parts within a work-group (1 or 2)
   int xs;           // key parts over work-groups (1: none), with a workspace
   int ks_plain;     // ks of the same call without a workspace (xs = 1)
@@ -52,6 +54,7 @@ PrefillShape prefill_shape(bool paged, bool fp8, int64_t batch, int64_t max_seql
   const int gqa = num_heads / num_kv_heads;
   const int hw = gqa < kPrefillWaves ? gqa : kPrefillWaves;  // query heads per work-group
   const int64_t wg_tokens = prefill_wg_tokens(gqa, head_size, head_size_v);
+  sh.wg_tokens = wg_tokens;
   sh.qblocks = (max_seqlen_q + wg_tokens - 1) / wg_tokens;
   sh.hsplit = (gqa + hw - 1) / hw;
   // Key split when the 4-wave launch would leave SIMDs with one wave: fewer
@@ -59,6 +62,7 @@ PrefillShape prefill_shape(bool paged, bool fp8, int64_t batch, int64_t max_seql
   // twice its queries pairs its blocks two per work-group; max_seqlen_k (a
   // bound on every sequence's keys, 0 = unknown) tells whether that can happen.
   const bool may_pair = causal && max_seqlen_k > 0 && max_seqlen_k < 2 * max_seqlen_q;
+  sh.may_pair = may_pair;
   const int64_t wgs = static_cast<int64_t>(num_kv_heads) * sh.hsplit * batch *
                       (may_pair ? (sh.qblocks + 1) / 2 : sh.qblocks);
   sh.ks = ((std::max(head_size, head_size_v) <= 192 || paged) && wgs < 2LL * num_cus()) ? 2 : 1;
@@ -147,6 +151,57 @@ PrefillShape prefill_shape(bool paged, bool fp8, int64_t batch, int64_t max_seql
     }
   }
   return sh;
+}
+
+// The launch's item order: the number of sequences for the kernel's longest-first order
+// (PrefillParams::lpt), or 0 for the grid's own (sequence by sequence, block index
+// slowest).  items: an upper bound of the launch's query blocks (pairs count twice).
+//
+// Longest first fills the tail of a ragged launch and leaves no gaps for the absent
+// blocks of its shorter sequences, but every work-group pays for finding its item, about
+// 0.045 us a sequence, and it takes a sequence's blocks together: at equal lengths the
+// light last blocks no longer come last, and where the grid's x is not a multiple of the
+// 8 XCDs a sequence's blocks read its keys through several L2s.  Measured on one box,
+// whole calls, us, own order / longest first (lengths uniform in the range given):
+//   equal lengths: 9 x 200 at 32 / 8 / 128 22 / 33, 64 x 100 39 / 48, 64 x 200 at 64 / 8 /
+//     64 80 / 119, 64 x 32 over 2000 at 16 / 2 / 256 113 / 170
+//   ragged and short: 64 x (4 .. 40) 14 / 19, a vision batch of 64 x (15 .. 60) 12.7 / 18.7
+//   ragged: 5 x (60 .. 600) 36 / 24, 16 x (150 .. 1500) 228 / 155, 16 x (75 .. 300) over
+//     (1000 .. 4000) 238 / 167, 2 x (150 .. 1500) 71 / 40
+//   ragged, many: 64 x (60 .. 600) 198 / 213, at 64 / 8 / 64 206 / 255
+//   equal lengths whose keys pass the caches: 64 x 200 over 1000 399 / 372, at 16 / 2 / 256
+//     507 / 378, 64 x 600 at 16 / 2 / 256 512 / 412
+// so it is taken when
+//   - the launch holds more work-groups than CUs (else each has a CU to itself in any
+//     order) of four stages or more, with long keys already at 3/4 of them, and
+//   - the lengths differ: the rows are fewer than 90 % of batch * max_seqlen_q (total_q 0:
+//     unknown, taken as ragged), and the search stays small against an item's stages: at
+//     most 9 stages for each sequence and round of the slots; or
+//   - over four rounds and more the batch's keys exceed what holds them: the last-level
+//     cache, or, where a work-group computes 64 rows for each key read (head size 256),
+//     the L2s.
+// Head 256 with one or two blocks a sequence in one round keeps its own order (the L2s).
+int prefill_order(const PrefillShape& sh, int xs, int64_t batch, int64_t total_q,
+                  int64_t max_seqlen_q, int64_t max_seqlen_k, int num_kv_heads, int head_size,
+                  int head_size_v, int window_left, int elem, int64_t items) {
+  if (batch > 64 || items * xs > 65535) return 0;
+  if (batch == 1) return 1;  // (its blocks in order, at no cost)
+  const double ncu = num_cus();
+  const double gx = static_cast<double>(num_kv_heads) * sh.hsplit * xs / (sh.may_pair ? 2 : 1);
+  double keys = static_cast<double>(std::max(max_seqlen_k, max_seqlen_q));
+  if (window_left >= 0)
+    keys = std::min(keys, static_cast<double>(window_left) + static_cast<double>(sh.wg_tokens));
+  const double stages = keys / kStageKeys;
+  const double wgs = gx * static_cast<double>(batch * sh.qblocks);  // absent blocks included
+  if (!(wgs > ncu * 9 / 8 && stages >= 4) && !(wgs > ncu * 3 / 4 && stages >= 32)) return 0;
+  const double rounds = gx * static_cast<double>(items) / (2 * ncu);
+  const bool few_rows = col_blocks_for(head_size, head_size_v) == 1;
+  const double key_bytes =
+      static_cast<double>(batch) * keys * num_kv_heads * (head_size + head_size_v) * elem;
+  if (rounds >= 4 && key_bytes > (few_rows ? 32e6 : 256e6)) return static_cast<int>(batch);
+  if (total_q > 0 && 10 * total_q > 9 * batch * max_seqlen_q) return 0;
+  if (few_rows && num_kv_heads * sh.hsplit % 8 != 0 && rounds <= 1 && sh.qblocks <= 2) return 0;
+  return batch * rounds <= 9 * stages ? static_cast<int>(batch) : 0;
 }
 
 // Bytes of the work-group key split's partial states (0 without the split).
@@ -356,13 +411,14 @@ int prefill_entry(const char* name, bool paged, void* out, int64_t out_row_strid
   P.num_heads = num_heads;
   FK_REQUIRE(qblocks <= 65535, "%s: max_seqlen_q %lld needs more than 65535 query blocks", name,
              (long long)max_seqlen_q);
-  // Longest items first: up to 64 sequences (one per lane of the kernel's ordering).
   // Items: at most ceil(q_len / block) per sequence, and with a workspace (whose size
   // total_q was already bounded by) no more than total_q rows hold.
-  const int64_t wg_tokens = prefill_wg_tokens(P.gqa, head_size, head_size_v);
   int64_t items = batch * qblocks;
-  if (workspace != nullptr && total_q > 0) items = std::min(items, total_q / wg_tokens + batch);
-  P.lpt = (batch <= 64 && items * sh.xs <= 65535) ? static_cast<int>(batch) : 0;
+  if (workspace != nullptr && total_q > 0)
+    items = std::min(items, total_q / sh.wg_tokens + batch);
+  P.lpt = prefill_order(sh, sh.xs, batch, workspace ? total_q : 0, max_seqlen_q, max_seqlen_k,
+                        num_kv_heads, head_size, head_size_v, window_left,
+                        static_cast<int>(elem), items);
   const dim3 grid =
       P.lpt ? dim3(static_cast<unsigned>(num_kv_heads * sh.hsplit),
                    static_cast<unsigned>(items * sh.xs), 1)
@@ -461,6 +517,38 @@ extern "C" int fk_prefill_split_plan(int paged, int kv_dtype, int64_t batch, int
       fk::prefill_shape(paged != 0, kv_dtype == FK_DTYPE_FP8_E4M3FN, batch, max_seqlen_q,
                         max_seqlen_k, num_heads, num_kv_heads, head_size, head_size_v, causal);
   *workspace_bytes = fk::prefill_ws_bytes(sh, total_q, num_heads, head_size_v);
+  return FK_OK;
+}
+
+extern "C" int fk_prefill_shape(int paged, int kv_dtype, int64_t batch, int64_t total_q,
+                                int64_t max_seqlen_q, int64_t max_seqlen_k, int num_heads,
+                                int num_kv_heads, int head_size, int head_size_v, int causal,
+                                int window_left, int with_workspace, int* wg_tokens,
+                                int* key_split, int* parts, int* longest_first) {
+  const char* name = "fk_prefill_shape";
+  FK_REQUIRE(wg_tokens && key_split && parts && longest_first, "%s: null output pointer", name);
+  FK_REQUIRE(batch > 0 && total_q >= 0 && max_seqlen_q > 0 && max_seqlen_k >= 0,
+             "%s: batch and max_seqlen_q must be positive", name);
+  FK_REQUIRE(num_heads > 0 && num_kv_heads > 0 && num_heads % num_kv_heads == 0,
+             "%s: num_heads %d must be a positive multiple of num_kv_heads %d", name, num_heads,
+             num_kv_heads);
+  const bool fp8 = kv_dtype == FK_DTYPE_FP8_E4M3FN;
+  fk::PrefillShape sh =
+      fk::prefill_shape(paged != 0, fp8, batch, max_seqlen_q, max_seqlen_k, num_heads,
+                        num_kv_heads, head_size, head_size_v, causal);
+  if (!with_workspace) {
+    sh.xs = 1;
+    sh.ks = sh.ks_plain;
+    total_q = 0;
+  }
+  int64_t items = batch * sh.qblocks;
+  if (total_q > 0) items = std::min(items, total_q / sh.wg_tokens + batch);
+  *wg_tokens = static_cast<int>(sh.wg_tokens);
+  *key_split = sh.ks;
+  *parts = sh.xs;
+  *longest_first =
+      fk::prefill_order(sh, sh.xs, batch, total_q, max_seqlen_q, max_seqlen_k, num_kv_heads,
+                        head_size, head_size_v, window_left, fp8 ? 1 : 2, items);
   return FK_OK;
 }
 

@@ -78,7 +78,7 @@ extern "C" {
  * header checks fk_version() / 10000 == FK_VERSION_MAJOR before binding. */
 #define FK_VERSION_MAJOR 2
 /* 2.1: fk_prefill_split_plan, fk_paged_prefill_ws, fk_varlen_prefill_ws
- * 2.2: fk_paged_decode_shape */
+ * 2.2: fk_paged_decode_shape, fk_prefill_shape */
 #define FK_VERSION_MINOR 2
 int fk_version(void);
 
@@ -338,6 +338,19 @@ int fk_prefill_split_plan(int paged, int kv_dtype, int64_t batch, int64_t total_
                           int64_t max_seqlen_q, int64_t max_seqlen_k, int num_heads,
                           int num_kv_heads, int head_size, int head_size_v, int causal,
                           int64_t* workspace_bytes);
+
+/* How the prefill entry points launch these sizes (host-only, for tests and profiling;
+ * arguments as fk_prefill_split_plan, with_workspace: 1 for the _ws entry points with
+ * one):
+ *   wg_tokens:     query tokens of a work-group.
+ *   key_split:     2 when the halves of a work-group divide its keys, else 1.
+ *   parts:         work-groups that divide each block's keys (1 without a workspace).
+ *   longest_first: 0 for the grid's own order, else the sequences ordered. */
+int fk_prefill_shape(int paged, int kv_dtype, int64_t batch, int64_t total_q,
+                     int64_t max_seqlen_q, int64_t max_seqlen_k, int num_heads, int num_kv_heads,
+                     int head_size, int head_size_v, int causal, int window_left,
+                     int with_workspace, int* wg_tokens, int* key_split, int* parts,
+                     int* longest_first);
 
 /* fk_paged_prefill / fk_varlen_prefill with the work-group key split's workspace:
  * workspace NULL runs exactly the entry point without _ws (total_q is ignored);

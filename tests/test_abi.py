@@ -181,6 +181,31 @@ def test_decode_work_groups_fit_the_kernel(lib):
     assert _native.decode_shape(100, 9, 3, 64, -1, 512, 4) == (4, 2, False)
 
 
+def test_prefill_order_rule(lib):
+    """fk_prefill_shape's item order: longest first for ragged launches that hold more
+    work-groups than CUs, the grid's own for equal or short lengths, small launches, more
+    than 64 sequences, and where the search would outweigh the items."""
+    from fastkernels_amd import _native as N
+
+    def order(batch, max_q, total_q, max_k=0, hq=32, hk=8, d=128, causal=True, window=-1, ws=True):
+        return N.prefill_shape(True, N.FK_DTYPE_BF16, batch, total_q, max_q, max_k or max_q, hq,
+                               hk, d, d, causal, window, ws)[3]
+
+    assert order(16, 1500, 13000) == 16          # ragged prompts
+    assert order(16, 1500, 16 * 1500) == 0       # equal ones
+    assert order(65, 1500, 50000) == 0           # past the ordering's 64
+    assert order(1, 1500, 1500) == 1             # one sequence: its blocks in order
+    assert order(64, 40, 1300) == 0              # short
+    assert order(64, 200, 7000) == 0             # many short ones: the search outweighs them
+    assert order(5, 200, 600) == 0               # fewer work-groups than CUs
+    assert order(16, 300, 3000, max_k=4300) == 16  # ragged chunks over long caches
+    assert order(16, 300, 3000, max_k=4300, window=10) == 0  # a short window: few stages
+    assert order(64, 200, 64 * 200, max_k=1200) == 64  # equal, keys past the last-level cache
+    assert order(64, 200, 64 * 200, max_k=300) == 0
+    assert order(64, 600, 64 * 600, hq=16, hk=2, d=256) == 64  # head 256: past the L2s
+    assert order(16, 1500, 0, ws=False) == 16    # rows unknown: taken as ragged
+
+
 def test_argument_errors_return_before_launch(lib):
     from fastkernels_amd import _native as N
 
