@@ -29,14 +29,15 @@ void launch_prefill_d(bool paged, bool fp8, bool split, const PrefillParams& P, 
 }
 
 // Query tokens per work-group.
-int64_t prefill_wg_tokens(int gqa, int head_size, int head_size_v) {
+int64_t prefill_wg_tokens(int gqa, int col_blocks) {
   const int hw = gqa < kPrefillWaves ? gqa : kPrefillWaves;
-  return static_cast<int64_t>(kPrefillWaves / hw) * 16 * col_blocks_for(head_size, head_size_v);
+  return static_cast<int64_t>(kPrefillWaves / hw) * 16 * col_blocks;
 }
 
 // Launch shape of a prefill call, from the host-side bounds alone (the plan
 // entry point and the launch agree on it).
 struct PrefillShape {
+  int col_blocks;     // 16-query column blocks per wave
   int64_t wg_tokens;  // query tokens per work-group
   int64_t qblocks;    // query blocks per sequence (grid z before the key parts)
   bool may_pair;      // causal pairs of blocks may occur
@@ -47,16 +48,46 @@ struct PrefillShape {
   bool part_f32;    // the key parts' O in fp32 rather than bf16
 };
 
-PrefillShape prefill_shape(bool paged, bool fp8, int64_t batch, int64_t max_seqlen_q,
-                           int64_t max_seqlen_k, int num_heads, int num_kv_heads, int head_size,
+// MLA's head sizes (one_col_block_built): two column blocks a wave, or one.  Two serve 32
+// queries with each K / V byte read from LDS but make half as many work-groups; with too
+// few of them CUs stay idle and each one's block takes longer.  Two where their
+// work-groups (a causal pair counts as one) pass 5/8 of the CUs, or their keys are long
+// enough that parts of them make up for it: 2^18 keys over all work-groups, twice that for
+// causal pairs, which see half.  A block of 128 of at most 64 queries would be half empty:
+// one.  Measured on one box, us, one / two (heads of 192 / 128):
+//   causal, 16 heads: 1x256 13.2 / 20.1, 1x1024 27 / 33, 1x2048 43 / 48, 4x512 20 / 27,
+//     32x33 7.3 / 8.8; 1x3000 111 / 75, 4x1024 42.2 / 39.5, 16x400 47 / 40
+//   not causal, 16 heads: 1x512 over 1024 22 / 26, 1x1024 over 1024 23 / 28; 1x512 over
+//     4096 44 / 39, 1x2000 over 2000 61 / 51, 8x200 over 1000 35 / 32; 128 heads: 4x256
+//     over 512 83 / 67, 8x200 over 1000 300 / 210
+bool two_col_blocks(int64_t batch, int64_t total_q, int64_t max_seqlen_q, int64_t max_seqlen_k,
+                    int64_t grid_x, int64_t wg_tokens, int causal) {
+  if (2 * max_seqlen_q <= wg_tokens) return false;
+  const bool pairs = causal && max_seqlen_k < 2 * max_seqlen_q;
+  int64_t blocks = batch * ((max_seqlen_q + wg_tokens - 1) / wg_tokens);
+  if (total_q > 0) blocks = std::min(blocks, total_q / wg_tokens + batch);
+  const int64_t wgs = grid_x * (pairs ? (blocks + 1) / 2 : blocks);
+  const int64_t keys = std::max(max_seqlen_k, max_seqlen_q);
+  return 8 * wgs >= 5LL * num_cus() || wgs * keys >= (int64_t(1) << (pairs ? 19 : 18));
+}
+
+// total_q: the rows of q, or 0 if unknown.
+PrefillShape prefill_shape(bool paged, bool fp8, int64_t batch, int64_t total_q,
+                           int64_t max_seqlen_q, int64_t max_seqlen_k, int num_heads, int num_kv_heads, int head_size,
                            int head_size_v, int causal) {
   PrefillShape sh;
   const int gqa = num_heads / num_kv_heads;
   const int hw = gqa < kPrefillWaves ? gqa : kPrefillWaves;  // query heads per work-group
-  const int64_t wg_tokens = prefill_wg_tokens(gqa, head_size, head_size_v);
+  sh.hsplit = (gqa + hw - 1) / hw;
+  sh.col_blocks = col_blocks_for(head_size, head_size_v);
+  if (one_col_block_built(head_size, head_size_v) &&
+      !two_col_blocks(batch, total_q, max_seqlen_q, max_seqlen_k,
+                      static_cast<int64_t>(num_kv_heads) * sh.hsplit,
+                      prefill_wg_tokens(gqa, 2), causal))
+    sh.col_blocks = 1;
+  const int64_t wg_tokens = prefill_wg_tokens(gqa, sh.col_blocks);
   sh.wg_tokens = wg_tokens;
   sh.qblocks = (max_seqlen_q + wg_tokens - 1) / wg_tokens;
-  sh.hsplit = (gqa + hw - 1) / hw;
   // Key split when the 4-wave launch would leave SIMDs with one wave: fewer
   // work-groups than two per CU.  A causal sequence with fewer cached keys than
   // twice its queries pairs its blocks two per work-group; max_seqlen_k (a
@@ -195,7 +226,7 @@ int prefill_order(const PrefillShape& sh, int xs, int64_t batch, int64_t total_q
   const double wgs = gx * static_cast<double>(batch * sh.qblocks);  // absent blocks included
   if (!(wgs > ncu * 9 / 8 && stages >= 4) && !(wgs > ncu * 3 / 4 && stages >= 32)) return 0;
   const double rounds = gx * static_cast<double>(items) / (2 * ncu);
-  const bool few_rows = col_blocks_for(head_size, head_size_v) == 1;
+  const bool few_rows = sh.col_blocks == 1;
   const double key_bytes =
       static_cast<double>(batch) * keys * num_kv_heads * (head_size + head_size_v) * elem;
   if (rounds >= 4 && key_bytes > (few_rows ? 32e6 : 256e6)) return static_cast<int>(batch);
@@ -367,8 +398,9 @@ int prefill_entry(const char* name, bool paged, void* out, int64_t out_row_strid
                  v_row_bytes % 16 == 0,
              "%s: q/out/keys/values must be 16-byte aligned with 16-byte row strides", name);
   const bool fp8 = kv_dtype == FK_DTYPE_FP8_E4M3FN;
-  PrefillShape sh = prefill_shape(paged, fp8, batch, max_seqlen_q, max_seqlen_k, num_heads,
-                                  num_kv_heads, head_size, head_size_v, causal);
+  PrefillShape sh = prefill_shape(paged, fp8, batch, workspace ? total_q : 0, max_seqlen_q,
+                                  max_seqlen_k, num_heads, num_kv_heads, head_size, head_size_v,
+                                  causal);
   if (workspace == nullptr) {
     sh.xs = 1;  // no workspace: the launch without the work-group key split
     sh.ks = sh.ks_plain;
@@ -409,6 +441,7 @@ int prefill_entry(const char* name, bool paged, void* out, int64_t out_row_strid
   P.part = workspace;
   P.part_rows = total_q;
   P.num_heads = num_heads;
+  P.col_blocks = sh.col_blocks;
   FK_REQUIRE(qblocks <= 65535, "%s: max_seqlen_q %lld needs more than 65535 query blocks", name,
              (long long)max_seqlen_q);
   // Items: at most ceil(q_len / block) per sequence, and with a workspace (whose size
@@ -514,7 +547,7 @@ extern "C" int fk_prefill_split_plan(int paged, int kv_dtype, int64_t batch, int
              num_kv_heads);
   if (batch == 0 || max_seqlen_q == 0 || total_q == 0) return FK_OK;
   const fk::PrefillShape sh =
-      fk::prefill_shape(paged != 0, kv_dtype == FK_DTYPE_FP8_E4M3FN, batch, max_seqlen_q,
+      fk::prefill_shape(paged != 0, kv_dtype == FK_DTYPE_FP8_E4M3FN, batch, total_q, max_seqlen_q,
                         max_seqlen_k, num_heads, num_kv_heads, head_size, head_size_v, causal);
   *workspace_bytes = fk::prefill_ws_bytes(sh, total_q, num_heads, head_size_v);
   return FK_OK;
@@ -534,7 +567,7 @@ extern "C" int fk_prefill_shape(int paged, int kv_dtype, int64_t batch, int64_t 
              num_kv_heads);
   const bool fp8 = kv_dtype == FK_DTYPE_FP8_E4M3FN;
   fk::PrefillShape sh =
-      fk::prefill_shape(paged != 0, fp8, batch, max_seqlen_q, max_seqlen_k, num_heads,
+      fk::prefill_shape(paged != 0, fp8, batch, with_workspace ? total_q : 0, max_seqlen_q, max_seqlen_k, num_heads,
                         num_kv_heads, head_size, head_size_v, causal);
   if (!with_workspace) {
     sh.xs = 1;

@@ -100,6 +100,7 @@ struct PrefillParams {
   // the item (sequence, query block or pair) in descending order of the
   // sequence's key stages (x P.xs key parts, the part fastest).
   int lpt;
+  int col_blocks;  // host only: 16-query column blocks per wave of the kernel to launch
 };
 
 // Floats of the partial state per (part, row, head) besides O.
@@ -148,11 +149,13 @@ constexpr float kFar = -1.0e30f;  // the max the exponent subtracts before a col
 constexpr int kQTokens = 16 * kColBlocks;      // query tokens per wave at head size 128
 // Column blocks per wave at head sizes (D, DV): at 256 the O accumulators of one
 // block (16 tiles of 4 fp32 per lane) already take what two take at 128.  MLA's
-// 192 / 128 takes two (246 registers): each K / V byte read from LDS then serves
-// 32 queries, and a work-group 128 instead of 64.  Same box, us: 877 and 1200 new
-// tokens over 2669 and 3300 cached ones, 16 heads (both calls and the merge) 249
-// -> 198; 300 .. 2000 over 500 .. 1500 178 -> 157; 1x256 over 8192 unchanged (64).
+// 192 / 128 takes two (246 registers): each K / V byte read from LDS then serves 32
+// queries, and a work-group 128 instead of 64; launches that this would leave short of
+// work-groups take one (two_col_blocks).
 constexpr int col_blocks_for(int D, int DV) { return (D > 192 || DV > 128) ? 1 : kColBlocks; }
+// Head sizes built with one column block too, for launches that two would leave short of
+// work-groups (prefill_shape's choice).
+constexpr bool one_col_block_built(int D, int DV) { return D > 128 && DV <= 128; }
 // MFMA extents: the score MFMAs run over D rounded up to 32, P.V over DV rounded
 // up to 16.
 constexpr int qk_extent(int D) { return (D + 31) / 32 * 32; }
@@ -425,7 +428,8 @@ __device__ __forceinline__ bool lpt_item(const PrefillParams& P, const int32_t* 
 // output is divided by is summed from the same bf16 P weights as the numerator
 // (an MFMA against ones); the log-sum-exp needs the exact sum, so it keeps an
 // fp32 sum of P per query column besides (8 adds per column block and 32 keys).
-template <bool kFp8, bool kPaged, int D, int DV, int kKS, bool kLse = false>
+template <bool kFp8, bool kPaged, int D, int DV, int kKS, bool kLse = false,
+          int kCB = col_blocks_for(D, DV)>  // kCB: 16-query column blocks per wave
 __global__ __launch_bounds__(kKS * kPrefillWaves * 64)
 __attribute__((amdgpu_waves_per_eu(kPrefillWavesPerSimd))) void
 paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
@@ -446,7 +450,6 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
   using SB = Stage<false, D, DV>;         // the layout the compute path reads
   static_assert(kKS == 1 || (kKS == 2 && (D <= 192 || kPaged)),
                 "key split: two halves, head size <= 192 (256 with paged keys)");
-  constexpr int kCB = col_blocks_for(D, DV);  // 16-query column blocks per wave
   constexpr int kQT = 16 * kCB;               // query tokens per wave
   constexpr int kDQ = qk_extent(D);           // score MFMA extent
   constexpr int kQC = kDQ / 32;               // score MFMAs per tile and column block
@@ -1461,18 +1464,31 @@ constexpr bool prefill_can_split(int D, int DV, bool paged) {
   return (D > DV ? D : DV) <= 192 || paged;
 }
 
-template <bool FP8, bool PAGED, int D, int DV, bool LSE>
-void launch_prefill_lse(bool split, const PrefillParams& P, dim3 grid, const int32_t* bt,
-                        const int32_t* cu_q, const int32_t* cu_k, hipStream_t stream) {
+template <bool FP8, bool PAGED, int D, int DV, bool LSE, int CB>
+void launch_prefill_cb(bool split, const PrefillParams& P, dim3 grid, const int32_t* bt,
+                       const int32_t* cu_q, const int32_t* cu_k, hipStream_t stream) {
   if constexpr (prefill_can_split(D, DV, PAGED)) {
     if (split) {
-      hipLaunchKernelGGL((paged_prefill_kernel<FP8, PAGED, D, DV, 2, LSE>), grid,
+      hipLaunchKernelGGL((paged_prefill_kernel<FP8, PAGED, D, DV, 2, LSE, CB>), grid,
                          dim3(2 * kPrefillWaves * 64), 0, stream, P, bt, cu_q, cu_k);
       return;
     }
   }
-  hipLaunchKernelGGL((paged_prefill_kernel<FP8, PAGED, D, DV, 1, LSE>), grid,
+  hipLaunchKernelGGL((paged_prefill_kernel<FP8, PAGED, D, DV, 1, LSE, CB>), grid,
                      dim3(kPrefillWaves * 64), 0, stream, P, bt, cu_q, cu_k);
+}
+
+template <bool FP8, bool PAGED, int D, int DV, bool LSE>
+void launch_prefill_lse(bool split, const PrefillParams& P, dim3 grid, const int32_t* bt,
+                        const int32_t* cu_q, const int32_t* cu_k, hipStream_t stream) {
+  if constexpr (one_col_block_built(D, DV)) {
+    if (P.col_blocks == 1) {
+      launch_prefill_cb<FP8, PAGED, D, DV, LSE, 1>(split, P, grid, bt, cu_q, cu_k, stream);
+      return;
+    }
+  }
+  launch_prefill_cb<FP8, PAGED, D, DV, LSE, col_blocks_for(D, DV)>(split, P, grid, bt, cu_q,
+                                                                   cu_k, stream);
 }
 
 // The log-sum-exp output is built for dense keys (FlashAttnVarlen's

@@ -143,18 +143,21 @@ def test_varlen_prefill_workgroup_key_split_lse(cuda, hq, hk, d, dv, causal):
 
 
 @pytest.mark.parametrize("hq,hk,d,dv,causal,nseq", [(8, 2, 128, 128, True, 4),
-                                                    (2, 2, 192, 128, False, 8),
+                                                    (2, 2, 192, 128, False, 16),
                                                     (4, 4, 80, 80, False, 8)])
 def test_varlen_prefill_key_parts_long_keys(cuda, hq, hk, d, dv, causal, nseq):
-    """Dense keys, 512-query chunks over 8192 keys (128 blocks): 4-wave work-groups with
-    each block's keys in parts over work-groups (in place of the 8-wave key split), with
-    the log-sum-exp output."""
+    """Dense keys, 512-query chunks over 8192 keys (128 work-groups): 4-wave work-groups
+    with each block's keys in parts over work-groups (in place of the 8-wave key split),
+    with the log-sum-exp output."""
     _flush(f"varlen key parts over 8192 keys {hq}/{hk}/{d}/{dv} causal={causal} x{nseq}")
     q_lens, k_lens = [512] * nseq, [8192] * nseq
     q, k, v, cu_q, cu_k = H._dense(cuda, q_lens, k_lens, hq, hk, d, dv, seed=470 + d)
     nbytes = _native.prefill_split_bytes(False, _native.FK_DTYPE_BF16, nseq, q.shape[0], 512,
                                          8192, hq, hk, d, dv, causal)
     assert nbytes > 0
+    _, key_split, parts, _ = _native.prefill_shape(False, _native.FK_DTYPE_BF16, nseq, q.shape[0],
+                                                   512, 8192, hq, hk, d, dv, causal)
+    assert key_split == 1 and parts > 1
     scale = d ** -0.5
     ref_o, ref_l = H._oracle_dense(q, k, v, cu_q, cu_k, scale, causal, lse=True)
     out, lse = H._run_dense(q, k, v, cu_q, cu_k, 512, scale, causal, lse=True, max_k=8192)
