@@ -183,7 +183,11 @@ struct DstConv<FK_DTYPE_FP8_E4M3FN> {
 template <>
 struct DstConv<FK_DTYPE_BF16> {
   using storage = uint16_t;
-  __device__ __forceinline__ static storage conv(float f) { return BF16::from_f32(f); }
+  // (The conversion instruction keeps a NaN's sign and payload; the cache holds the one
+  // quiet NaN, as torch's cast gives.)
+  __device__ __forceinline__ static storage conv(float f) {
+    return f != f ? static_cast<storage>(0x7fc0) : BF16::from_f32(f);
+  }
 };
 template <>
 struct DstConv<FK_DTYPE_F16> {

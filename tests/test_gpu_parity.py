@@ -1000,6 +1000,28 @@ def test_store_kvcache_convert_to_fp8(cuda, src):
     assert np.array_equal(vc_d.view(torch.uint8).cpu().numpy().reshape(-1, hk * d), zv)
 
 
+def test_store_kvcache_convert_f32_to_bf16_bits(cuda):
+    """Every fp32 sign, exponent and upper mantissa with lower halves around the rounding
+    points, against the rounding written out on integers: nearest even, subnormals kept,
+    every NaN the quiet 0x7fc0."""
+    _flush("store_kvcache convert f32 -> bf16, bits")
+    hi = torch.arange(1 << 16, dtype=torch.int64)[:, None] << 16
+    lo = torch.tensor([0, 1, 0x7fff, 0x8000, 0x8001, 0xc000, 0xfffe, 0xffff])
+    u = (hi | lo).view(-1)
+    want = ((u + 0x7fff + ((u >> 16) & 1)) >> 16) & 0xffff
+    want[(u & 0x7fffffff) > 0x7f800000] = 0x7fc0
+    key = torch.where(u >= 1 << 31, u - (1 << 32), u).to(torch.int32).to(cuda)
+    key = key.view(torch.float32).view(-1, 8, 128)
+    n = key.shape[0]
+    kc = torch.zeros(n // 16, 16, 8, 128, dtype=torch.bfloat16, device=cuda)
+    vc = torch.zeros_like(kc)
+    ops.store_kvcache(key, key, kc, vc, torch.arange(n, device=cuda))
+    torch.cuda.synchronize()
+    for c in (kc, vc):
+        got = c.view(torch.int16).view(-1).cpu().to(torch.int64) & 0xffff
+        assert torch.equal(got, want)
+
+
 def test_store_kvcache_convert_f32_to_bf16(cuda):
     g = torch.Generator().manual_seed(91)
     key = torch.randn(33, 2, 64, generator=g).to(cuda)
