@@ -271,8 +271,9 @@ def qk_norm_rope_store(positions: torch.Tensor, query: torch.Tensor, key: torch.
     tokens = positions.numel()
     dtype = query.dtype
     if not (key.dtype == value.dtype == k_cache.dtype == v_cache.dtype == dtype):
-        raise TypeError("qk_norm_rope_store: the key, value, k_cache and v_cache dtypes must "
-                        "equal the query dtype")
+        for t, nm in ((key, "key"), (value, "value"), (k_cache, "k_cache"), (v_cache, "v_cache")):
+            if t.dtype != dtype:
+                raise TypeError(f"qk_norm_rope_store: {nm} dtype must equal the query dtype")
     cs_dtype = cos_sin_cache.dtype
     if cos_sin_cache.dim() != 2 or not cos_sin_cache.is_contiguous() or \
             (cs_dtype != torch.float32 and cs_dtype != dtype):

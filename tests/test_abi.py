@@ -260,6 +260,23 @@ def test_python_layer_fails_loudly_without_gpu(lib):
         ops.rms_norm(torch.empty(4, 64), torch.zeros(4, 64), torch.ones(64), 1e-6)
 
 
+@pytest.mark.parametrize("wrong", ["key", "value", "k_cache", "v_cache"])
+def test_qk_norm_rope_store_names_the_wrong_dtype(lib, wrong):
+    import torch
+
+    from fastkernels_amd import ops
+
+    bf16 = dict(dtype=torch.bfloat16)
+    t = dict(query=torch.zeros(2, 256, **bf16), key=torch.zeros(2, 128, **bf16),
+             value=torch.zeros(2, 128, **bf16), k_cache=torch.zeros(1, 16, 2, 64, **bf16),
+             v_cache=torch.zeros(1, 16, 2, 64, **bf16))
+    t[wrong] = t[wrong].float()
+    with pytest.raises(TypeError, match=rf"qk_norm_rope_store: {wrong} dtype"):
+        ops.qk_norm_rope_store(torch.zeros(2, dtype=torch.int64), t["query"], t["key"], t["value"],
+                               t["k_cache"], t["v_cache"], torch.zeros(2, dtype=torch.int64), 64,
+                               torch.zeros(8, 64), True)
+
+
 def test_missing_library_raises(monkeypatch, tmp_path):
     from fastkernels_amd import _native
 
