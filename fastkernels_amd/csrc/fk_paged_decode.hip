@@ -50,13 +50,10 @@
 // stays at a few instructions (no cross-lane dot-product reductions, two
 // row-swap permutes per tile for the max).
 //
-// Two alternative tile forms are compiled in only for A/B measurement; the
-// shipped library defines neither macro, and both measured slower on C3:
+// An alternative tile form is compiled in only for A/B measurement; the shipped library
+// does not define its macro, and it measured slower on C3:
 //   FK_DECODE_VALU_TILE  bf16, head size 128, groups of up to 4 query heads:
 //     Q K^T and P V on the VALU (v_dot2_f32_bf16) instead of the matrix cores.
-//   FK_DECODE_LDS_STAGE  bf16, head size 128, plain decode: K/V tiles go from
-//     HBM straight to LDS (global_load_lds_dwordx4) through a two-stage ring
-//     per wave, so the next tile's loads are in flight while a tile is used.
 #include <limits.h>
 
 #include "fk_attn_tile.h"
@@ -80,11 +77,6 @@ namespace {
 constexpr bool kValuBuild = true;
 #else
 constexpr bool kValuBuild = false;
-#endif
-#ifdef FK_DECODE_LDS_STAGE
-constexpr bool kLdsBuild = true;
-#else
-constexpr bool kLdsBuild = false;
 #endif
 
 struct DecodeParams {
@@ -275,7 +267,7 @@ __device__ __forceinline__ void store_new_row(const DecodeParams& P, int b, int 
 }
 
 // ---------------------------------------------------------------------------
-// Helpers of the A/B tile forms (FK_DECODE_VALU_TILE, FK_DECODE_LDS_STAGE).
+// Helpers of the A/B tile form (FK_DECODE_VALU_TILE).
 // ---------------------------------------------------------------------------
 // DPP row reductions over the 16 lanes of each row: quad_perm [1,0,3,2] and
 // [2,3,0,1], then row_half_mirror and row_mirror; every lane gets the result.
@@ -308,28 +300,6 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
 __device__ __forceinline__ uint32_t lane_word(uint32_t v, int src) {
   return static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(src << 2, static_cast<int>(v)));
 }
-// 16 bytes from global memory straight into LDS: lane l writes at lds_addr +
-// 16 l.  Inline asm, so the compiler's wait-count pass does not track it; the
-// ring below orders it with explicit s_waitcnt.  M0 carries the LDS address
-// and is restored afterwards.
-__device__ __forceinline__ void lds_dma16(const uint8_t* src, uint32_t lds_addr) {
-  uint32_t saved;
-  asm volatile(
-      "s_mov_b32 %0, m0\n\t"
-      "s_mov_b32 m0, %2\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %1, off\n\t"
-      "s_nop 0\n\t"
-      "s_mov_b32 m0, %0"
-      : "=&s"(saved)
-      : "v"(src), "s"(lds_addr)
-      : "memory");
-}
-__device__ __forceinline__ uint32_t lds_addr_of(const uint8_t* p) {
-  return static_cast<uint32_t>(
-      reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const uint8_t*)p));
-}
-constexpr int kStageBytes = 8192;  // one bf16 tile at head size 128: K 4 KiB, then V 4 KiB
 
 // Online-softmax state of one wave over the query heads of one virtual head,
 // and the tile loop that streams a token range [tok_begin, tok_end) of a
@@ -339,10 +309,8 @@ template <int kG, int D, bool kFp8, int U, bool kStore>
 struct WaveState {
   static constexpr int kKc = D / 32;  // K chunks per row (QK^T MFMAs per tile)
   static constexpr int kSl = D / 16;  // P.V slices; also dims per lane
-  // A/B forms (off in the shipped build).
+  // A/B form (off in the shipped build).
   static constexpr bool kValu = kValuBuild && !kFp8 && D == 128 && kG == 4;
-  static constexpr bool kLds = kLdsBuild && !kFp8 && D == 128 && !kStore;
-  uint8_t* ring;  // kLds: this wave's two LDS stages
   float m_run;  // running max of column r (same in the 4 lanes of a column)
   float l_run;  // this lane's share of the running sum of column r
   float vsc;    // V's fp8 dequant scale of the kv head (1 for bf16 pages or no scale tensor)
@@ -360,7 +328,7 @@ struct WaveState {
                                       int tok_begin, int tok_end, int ctx, int key_lo, int r,
                                       int g, bool idle, bool lockstep = true) {
     constexpr int kSyncChunks = kFp8 ? FK_DECODE_SYNC_CHUNKS_FP8 : FK_DECODE_SYNC_CHUNKS;
-    constexpr bool kSync = kSyncChunks > 0 && !kLds;
+    constexpr bool kSync = kSyncChunks > 0;
     if (idle) {
       if (kSync && lockstep) {
         const int n = (tok_end - tok_begin + kTile - 1) / kTile;
@@ -593,24 +561,20 @@ struct WaveState {
     };
     // Chunks of U tiles: issue all U tiles' loads, then consume them in order
     // (the compiler waits for tile u with vmcnt = loads issued after it).
-    if constexpr (kLds) {
-      run_lds_ring(P, bt, b, kvh, tok_begin, ntiles, r, g, pc_idx, pc_page, process);
-    } else {
-      for (int t0 = 0, c = 0; t0 < ntiles; t0 += U, ++c) {
-        // Lock step (no wait for memory: gfx950's barrier does not drain the
-        // loads in flight).
-        if constexpr (kSync) {
-          if (lockstep && c % kSyncChunks == 0) __builtin_amdgcn_s_barrier();
-        }
-        if constexpr (kStore) {
-          if (t_store >= t0 && t_store < t0 + U && new_slot >= 0)
-            store_new_chunk<kFp8, D>(P, new_slot, kvh, 16 * g + r, new_chunk);
-        }
-        DTile<kFp8, D> buf[U];
-        int64_t pg[U];
-        fetch(t0, buf, pg);
-        consume(t0, buf, pg);
+    for (int t0 = 0, c = 0; t0 < ntiles; t0 += U, ++c) {
+      // Lock step (no wait for memory: gfx950's barrier does not drain the
+      // loads in flight).
+      if constexpr (kSync) {
+        if (lockstep && c % kSyncChunks == 0) __builtin_amdgcn_s_barrier();
       }
+      if constexpr (kStore) {
+        if (t_store >= t0 && t_store < t0 + U && new_slot >= 0)
+          store_new_chunk<kFp8, D>(P, new_slot, kvh, 16 * g + r, new_chunk);
+      }
+      DTile<kFp8, D> buf[U];
+      int64_t pg[U];
+      fetch(t0, buf, pg);
+      consume(t0, buf, pg);
     }
     if constexpr (kValu) {
       // Sum O over the 4 lane groups: lanes of group 0 then hold the MFMA
@@ -629,73 +593,6 @@ struct WaveState {
       // Column sums of l over the 4 lane groups: every lane of column j holds l_j.
       l_run = pair_sum(l_run);
     }
-  }
-
-  // kLds tile loop: tile t is staged in ring stage t % 2, tile t + 1's 8 loads
-  // are issued before tile t is waited for, read from LDS and processed.
-  // Tiles past the end re-read the last tile, so every wait is vmcnt(8).
-  template <typename Process>
-  __device__ __forceinline__ void run_lds_ring(const DecodeParams& P,
-                                               const int32_t* __restrict__ bt, int b, int kvh,
-                                               int tok_begin, int ntiles, int r, int g,
-                                               int& pc_idx, int64_t& pc_page, Process& process) {
-    const int lane = 16 * g + r;
-    const uint32_t ring_addr = __builtin_amdgcn_readfirstlane(lds_addr_of(ring));
-    const int64_t row_bytes = static_cast<int64_t>(P.num_kv_heads) * D * 2;
-    const int64_t head_off = static_cast<int64_t>(kvh) * D * 2;
-    auto issue = [&](int t, int stage) -> int64_t {
-      const int tok0 = tok_begin + kTile * min(t, ntiles - 1);
-      const int idx = tok0 >> P.block_size_log2;
-      if (idx != pc_idx) {
-        pc_page = page_of(P, bt, b, tok0);
-        pc_idx = idx;
-      }
-      const int64_t page = pc_page < 0 ? 0 : pc_page;
-      const int64_t slot0 = (page << P.block_size_log2) + (tok0 & ((1 << P.block_size_log2) - 1));
-      const uint8_t* krow = P.k_cache + (slot0 + r) * row_bytes + head_off;
-      const uint32_t base = ring_addr + stage * kStageBytes;
-#pragma unroll
-      for (int c = 0; c < 4; ++c) lds_dma16(krow + (32 * c + 8 * g) * 2, base + 1024 * c);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        lds_dma16(P.v_cache + (slot0 + 4 * g + i) * row_bytes + head_off + 16 * r,
-                  base + 4096 + 1024 * i);
-      return pc_page;
-    };
-    auto read = [&](int stage, DTile<kFp8, D>& t) {
-      const uint8_t* p = ring + stage * kStageBytes + 16 * lane;
-#pragma unroll
-      for (int c = 0; c < 4; ++c) t.k[c] = *reinterpret_cast<const uint4*>(p + 1024 * c);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const uint4 x = *reinterpret_cast<const uint4*>(p + 4096 + 1024 * i);
-        t.v[i][0] = x.x;
-        t.v[i][1] = x.y;
-        t.v[i][2] = x.z;
-        t.v[i][3] = x.w;
-      }
-    };
-    int64_t pg0 = issue(0, 0), pg1 = -1;
-    for (int t = 0; t < ntiles; t += 2) {
-      pg1 = issue(t + 1, 1);
-      asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-      {
-        DTile<kFp8, D> cur;
-        read(0, cur);
-        process(tok_begin + kTile * t, pg0, cur);
-      }
-      if (t + 1 >= ntiles) break;
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // stage 0's reads are done
-      pg0 = issue(t + 2, 0);
-      asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-      {
-        DTile<kFp8, D> cur;
-        read(1, cur);
-        process(tok_begin + kTile * (t + 1), pg1, cur);
-      }
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // stage 1's reads are done
-    }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the ring is free for the next segment
   }
 
   // Normalised output rows of the virtual head for a sequence finished in place.
@@ -824,8 +721,6 @@ __attribute__((amdgpu_waves_per_eu(FK_DECODE_WAVES_PER_EU))) void paged_decode_p
     const int lo = key_lo(P, ctx);
     using WS = WaveState<kG, D, kFp8, U, kStore>;
     WS st;
-    __shared__ __align__(16) uint8_t ring[WS::kLds ? NH * 2 * kStageBytes : 16];
-    st.ring = ring + wave * 2 * kStageBytes;
     const int seg_begin = max(tok_begin, lo & ~(kTile - 1));
     if (P.split == 1) {
       st.run(P, block_tables, slot_mapping, b, vh, seg_begin, tok_end, ctx, lo, r, g, idle);
@@ -956,8 +851,6 @@ __attribute__((amdgpu_waves_per_eu(FK_DECODE_WAVES_PER_EU))) void paged_decode_b
     }
     using WS = WaveState<kG, D, kFp8, U, kStore>;
     WS st;
-    __shared__ __align__(16) uint8_t ring[WS::kLds ? NH * 2 * kStageBytes : 16];
-    st.ring = ring + wave * 2 * kStageBytes;
     for (int b = lo; b < batch && toff[b] < t_hi; ++b) {
       const int s_lo = max(t_lo, toff[b]) - toff[b];
       const int s_hi = min(t_hi, toff[b + 1]) - toff[b];
