@@ -46,8 +46,8 @@ _SIGNATURES = {
                                      c_int64, c_void_p]),
     "fk_paged_decode_plan": (c_int, [c_int64, c_int, c_int, c_int, c_int64, c_int,
                                      c_void_p, c_void_p, c_void_p]),
-    "fk_paged_decode_shape": (c_int, [c_int64, c_int, c_int, c_int, c_int, c_int64, c_int64,
-                                      c_void_p, c_void_p, c_void_p]),
+    "fk_paged_decode_shape": (c_int, [c_int64, c_int, c_int, c_int, c_int, c_int, c_int64,
+                                      c_int64, c_void_p, c_void_p, c_void_p]),
     "fk_paged_decode": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_int,
                                 c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_int,
                                 c_int, c_int, c_int, c_int64, c_float, c_int, c_void_p,
@@ -196,10 +196,10 @@ def plan(batch: int, num_heads: int, num_kv_heads: int, head_size: int, max_seq_
     return tuple(out)
 
 
-def decode_shape(batch: int, num_heads: int, num_kv_heads: int, head_size: int, window_left: int,
-                 part_tokens: int, max_parts: int) -> tuple[int, int, bool]:
+def decode_shape(batch: int, num_heads: int, num_kv_heads: int, head_size: int, kv_dtype: int,
+                 window_left: int, part_tokens: int, max_parts: int) -> tuple[int, int, bool]:
     """fk_paged_decode_shape: (waves, shares, whole_windows) of a plan's launch."""
     out = (c_int * 3)()
-    call("fk_paged_decode_shape", batch, num_heads, num_kv_heads, head_size, window_left,
+    call("fk_paged_decode_shape", batch, num_heads, num_kv_heads, head_size, kv_dtype, window_left,
          part_tokens, max_parts, ctypes.byref(out), ctypes.byref(out, 4), ctypes.byref(out, 8))
     return out[0], out[1], bool(out[2])

@@ -70,9 +70,10 @@ __device__ __forceinline__ uint2 fp8x4_to_bf16x4(uint32_t w) {
 }
 
 // The same values by way of fp32, four instructions instead of two.  K at head size 128
-// takes it: 64 / 8 / 128 heads, fp8 pages, us, two -> four instructions: 16 x (1333 ..
-// 4000) 28.4 -> 27.2, 4 x (5333 .. 16000) 29.5 -> 28.7, 16 x (5333 .. 16000) 78.9 ->
-// 79.4; at 64 and 256 four cost 5 to 10 % of the long contexts.
+// takes it under the balanced decode schedule: 64 / 8 / 128 heads, fp8 pages, us, two ->
+// four instructions: 16 x (1333 .. 4000) 28.4 -> 27.2, 4 x (5333 .. 16000) 29.5 -> 28.7, 16 x
+// (5333 .. 16000) 78.9 -> 79.4; at 64 and 256 four cost 5 to 10 % of the long contexts, and
+// in short whole windows up to 6 %.
 __device__ __forceinline__ uint2 fp8x4_to_bf16x4_by_f32(uint32_t w) {
   const auto lo = __builtin_amdgcn_cvt_pk_f32_fp8(w, false);
   const auto hi = __builtin_amdgcn_cvt_pk_f32_fp8(w, true);
@@ -195,8 +196,8 @@ struct DTile {
 };
 
 // K operand chunks (bf16, dims as described at DTile) of a loaded tile; fp8
-// bytes are converted exactly (fp8x4_to_bf16x4).
-template <bool kFp8, int D>
+// bytes are converted exactly (fp8x4_to_bf16x4, or with kByF32 through fp32).
+template <bool kByF32, bool kFp8, int D>
 __device__ __forceinline__ void k_chunks_d(const DTile<kFp8, D>& t, uint4 (&kc)[D / 32]) {
   if constexpr (!kFp8) {
 #pragma unroll
@@ -208,8 +209,8 @@ __device__ __forceinline__ void k_chunks_d(const DTile<kFp8, D>& t, uint4 (&kc)[
       const uint4& src = t.k[c >> 1];
       const uint32_t w0 = (c & 1) ? src.z : src.x;
       const uint32_t w1 = (c & 1) ? src.w : src.y;
-      const uint2 lo = D == 128 ? fp8x4_to_bf16x4_by_f32(w0) : fp8x4_to_bf16x4(w0);
-      const uint2 hi = D == 128 ? fp8x4_to_bf16x4_by_f32(w1) : fp8x4_to_bf16x4(w1);
+      const uint2 lo = kByF32 ? fp8x4_to_bf16x4_by_f32(w0) : fp8x4_to_bf16x4(w0);
+      const uint2 hi = kByF32 ? fp8x4_to_bf16x4_by_f32(w1) : fp8x4_to_bf16x4(w1);
       kc[c] = make_uint4(lo.x, lo.y, hi.x, hi.y);
     }
   }

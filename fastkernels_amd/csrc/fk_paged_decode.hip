@@ -305,7 +305,8 @@ __device__ __forceinline__ uint32_t lane_word(uint32_t v, int src) {
 // and the tile loop that streams a token range [tok_begin, tok_end) of a
 // sequence through it (tok_begin a multiple of 16).  Lane (r, g) of the O
 // accumulators holds O[column 4g + i][dims (D/16) r .. (D/16) r + D/16 - 1].
-template <int kG, int D, bool kFp8, int U, bool kStore>
+// kBalanced: the balanced schedule's (it picks the fp8 conversion of K).
+template <int kG, int D, bool kFp8, int U, bool kStore, bool kBalanced>
 struct WaveState {
   static constexpr int kKc = D / 32;  // K chunks per row (QK^T MFMAs per tile)
   static constexpr int kSl = D / 16;  // P.V slices; also dims per lane
@@ -468,7 +469,7 @@ struct WaveState {
         return;
       }
       uint4 kc[kKc];
-      k_chunks_d(cur, kc);
+      k_chunks_d<kBalanced && D == 128>(cur, kc);
       const floatx4_t acc = qk_scores_n(kc, qb);
       // A tile wholly inside the visible keys on a readable page (every tile but
       // those at a segment's edges) needs no mask: one wave-uniform test skips
@@ -719,7 +720,7 @@ __attribute__((amdgpu_waves_per_eu(FK_DECODE_WAVES_PER_EU))) void paged_decode_p
     // window's first key; one wholly before it streams nothing and leaves an
     // empty partial (max -inf, sum 0).
     const int lo = key_lo(P, ctx);
-    using WS = WaveState<kG, D, kFp8, U, kStore>;
+    using WS = WaveState<kG, D, kFp8, U, kStore, false>;
     WS st;
     const int seg_begin = max(tok_begin, lo & ~(kTile - 1));
     if (P.split == 1) {
@@ -849,7 +850,7 @@ __attribute__((amdgpu_waves_per_eu(FK_DECODE_WAVES_PER_EU))) void paged_decode_b
       const int mid = (lo + hi) >> 1;
       if (toff[mid] <= t_lo) lo = mid; else hi = mid;
     }
-    using WS = WaveState<kG, D, kFp8, U, kStore>;
+    using WS = WaveState<kG, D, kFp8, U, kStore, true>;
     WS st;
     for (int b = lo; b < batch && toff[b] < t_hi; ++b) {
       const int s_lo = max(t_lo, toff[b]) - toff[b];
@@ -1234,7 +1235,11 @@ int validate(const char* name, int64_t batch, int num_heads, int num_kv_heads, i
 // tiles a wave; where even the most do not fill it, they still run when a wave
 // has at most kSoloShort tiles (the balanced schedule's two launches cost more
 // than such a chain).  Returns 0 for the balanced schedule, which also evens out
-// long windows that only some of the sequences fill.  Kernel times on one box,
+// long windows that only some of the sequences fill.  fp8 pages take eight shares only up
+// to two work-groups per CU: a share then streams half the bytes, and over more rounds
+// the merges cost more than the balanced schedule's (window 1023, us, balanced -> eight
+// shares: 20 / 20 / 64 batch 64 41 -> 52, 160 107 -> 118, 32 / 8 / 128 batch 160 68 -> 73; 64
+// 32.4 -> 29.4, 8 / 1 / 128 batch 160 21 -> 15).  Kernel times on one box,
 // us, balanced (with its merge) -> whole windows, contexts 300 .. 6000: 64 / 8 / 64
 // heads, window 128, batch 16 12.5 -> 7.4, 128 29 -> 14, 256 55 -> 18; 32 / 8 / 128,
 // window 1024, batch 32 30.4 -> 24.5, 64 48.2 -> 45.5, window 512, batch 128 53.1
@@ -1246,12 +1251,13 @@ size_t solo_lds(int nh, int shares, int head_size) {
   return static_cast<size_t>(shares - 1) * nh * (head_size / 16 * 4 * 64 + 2 * 64) *
          sizeof(float);
 }
-int solo_shares(int64_t batch, int vheads, int head_size, int window_left) {
+int solo_shares(int64_t batch, int vheads, int head_size, bool fp8, int window_left) {
   if (window_left < 0 || window_left > (1 << 20)) return 0;
   const int tiles = (window_left + kTile) / kTile + 1;
   int most = 1;
   for (int s = 1; s <= kMaxWavesPerGroup && solo_lds(1, s, head_size) <= kSoloLds; s *= 2) {
-    if (batch * vheads * s >= kSoloWaves && tiles <= s * kSoloTiles) return s;
+    if (batch * vheads * s >= kSoloWaves && tiles <= s * kSoloTiles)
+      return fp8 && s == 8 && batch * vheads > 2LL * num_cus() ? 0 : s;
     most = s;
   }
   return tiles <= most * kSoloShort ? most : 0;
@@ -1267,14 +1273,14 @@ struct DecodeShape {
   int shares;
   size_t lds;
 };
-DecodeShape decode_shape(int64_t batch, int vheads, int head_size, int window_left,
+DecodeShape decode_shape(int64_t batch, int vheads, int head_size, bool fp8, int window_left,
                          int64_t part_tokens, int64_t max_parts) {
   const bool balanced = part_tokens == 0;
   // Rounded up to a power of two: 3 heads run as 4 waves with one idle.
   int p2 = 1;
   while (p2 < waves_per_group(vheads)) p2 *= 2;
   DecodeShape sh = {false, p2, 1, 0};
-  if (const int s = balanced ? solo_shares(batch, vheads, head_size, window_left) : 0) {
+  if (const int s = balanced ? solo_shares(batch, vheads, head_size, fp8, window_left) : 0) {
     // Work-groups of 8 waves or fewer whose states fit in 64 KB of LDS.
     sh.whole = true;
     sh.shares = s;
@@ -1384,7 +1390,8 @@ int prepare(const char* name, Launch& L, void* out, int64_t out_row_stride, cons
   L.fp8 = kv_dtype == FK_DTYPE_FP8_E4M3FN;
   L.head_size = head_size;
   const int vh = virtual_heads(num_heads, num_kv_heads);
-  const DecodeShape sh = decode_shape(batch, vh, head_size, window_left, part_tokens, max_parts);
+  const DecodeShape sh = decode_shape(batch, vh, head_size, L.fp8, window_left, part_tokens,
+                                      max_parts);
   L.nh = sh.waves;
   L.part_lds = sh.lds;
   P.split = sh.shares;
@@ -1549,15 +1556,16 @@ extern "C" int fk_paged_decode_plan(int64_t batch, int num_heads, int num_kv_hea
 }
 
 extern "C" int fk_paged_decode_shape(int64_t batch, int num_heads, int num_kv_heads,
-                                     int head_size, int window_left, int64_t part_tokens,
-                                     int64_t max_parts, int* waves, int* shares,
-                                     int* whole_windows) {
+                                     int head_size, int kv_dtype, int window_left,
+                                     int64_t part_tokens, int64_t max_parts, int* waves,
+                                     int* shares, int* whole_windows) {
   const char* name = "fk_paged_decode_shape";
   FK_REQUIRE(waves && shares && whole_windows, "%s: null output pointer", name);
   const int rc = validate(name, batch, num_heads, num_kv_heads, head_size, part_tokens, max_parts);
   if (rc != FK_OK) return rc;
   const DecodeShape sh = decode_shape(batch, virtual_heads(num_heads, num_kv_heads), head_size,
-                                      window_left, part_tokens, max_parts);
+                                      kv_dtype == FK_DTYPE_FP8_E4M3FN, window_left, part_tokens,
+                                      max_parts);
   *waves = sh.waves;
   *shares = sh.shares;
   *whole_windows = sh.whole ? 1 : 0;

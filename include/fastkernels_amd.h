@@ -167,8 +167,8 @@ int fk_paged_decode_plan(int64_t batch, int num_heads, int num_kv_heads, int hea
  *   whole_windows: 1 when, under a sliding window, a work-group takes each sequence's
  *                  whole window (no merge launch). */
 int fk_paged_decode_shape(int64_t batch, int num_heads, int num_kv_heads, int head_size,
-                          int window_left, int64_t part_tokens, int64_t max_parts, int* waves,
-                          int* shares, int* whole_windows);
+                          int kv_dtype, int window_left, int64_t part_tokens, int64_t max_parts,
+                          int* waves, int* shares, int* whole_windows);
 
 /* Paged decode attention (one query token per sequence, at position ctx_lens[b] - 1):
  *   out[b,h,:] = softmax(scale * q[b,h,:] . K_b^T) V_b  over tokens [lo_b, ctx_lens[b])

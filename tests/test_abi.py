@@ -168,17 +168,22 @@ def test_decode_work_groups_fit_the_kernel(lib):
                     for part, parts, window in ((512, 1, -1), (512, 4, -1), (512, 16, 100),
                                                 (0, 256, -1), (0, 256, 0), (0, 256, 127),
                                                 (0, 256, 1023), (0, 256, 5000)):
-                        waves, shares, whole = _native.decode_shape(batch, hk * group, hk, d,
-                                                                    window, part, parts)
-                        what = (batch, hk * group, hk, d, window, part, parts)
-                        assert waves in (1, 2, 4, 8) and shares in (1, 2, 4, 8), what
-                        assert waves * shares <= 8, what
-                        assert whole <= (part == 0 and window >= 0), what
-                        assert shares == 1 or whole or part > 0, what
-                        shares_seen.add((whole, shares))
+                        for kv in (_native.FK_DTYPE_BF16, _native.FK_DTYPE_FP8_E4M3FN):
+                            what = (batch, hk * group, hk, d, kv, window, part, parts)
+                            waves, shares, whole = _native.decode_shape(*what)
+                            assert waves in (1, 2, 4, 8) and shares in (1, 2, 4, 8), what
+                            assert waves * shares <= 8, what
+                            assert whole <= (part == 0 and window >= 0), what
+                            assert shares == 1 or whole or part > 0, what
+                            shares_seen.add((whole, shares))
     assert shares_seen == {(False, 1), (False, 2), (True, 1), (True, 2), (True, 4), (True, 8)}
     # The shape that made the illegal work-group: 3 kv heads, 100 sequences, 4 partitions.
-    assert _native.decode_shape(100, 9, 3, 64, -1, 512, 4) == (4, 2, False)
+    bf16, fp8 = _native.FK_DTYPE_BF16, _native.FK_DTYPE_FP8_E4M3FN
+    assert _native.decode_shape(100, 9, 3, 64, bf16, -1, 512, 4) == (4, 2, False)
+    # Eight shares over fp8 pages: up to two work-groups per CU (256 without a GPU).
+    assert _native.decode_shape(64, 32, 8, 128, fp8, 1023, 0, 256) == (1, 8, True)
+    assert _native.decode_shape(65, 32, 8, 128, fp8, 1023, 0, 256)[2] is False
+    assert _native.decode_shape(65, 32, 8, 128, bf16, 1023, 0, 256) == (1, 8, True)
 
 
 def test_prefill_order_rule(lib):
