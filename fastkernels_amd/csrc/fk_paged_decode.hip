@@ -1228,7 +1228,8 @@ int validate(const char* name, int64_t batch, int num_heads, int num_kv_heads, i
 }
 
 // Whole windows.  Under a sliding window a sequence streams at most
-// (window_left + 16) / 16 + 1 tiles, whatever its context, so a batch can give
+// (window_left + 16) / 16 + 1 tiles, whatever its context (one fewer where window_left
+// is a multiple of 16: the thresholds below were measured on this count), so a batch can give
 // each sequence to one work-group, each virtual head's tiles in `shares` (1, 2, 4
 // or 8) over as many waves that merge in LDS, with no merge launch.  The fewest
 // shares are taken that fill the chip (kSoloWaves waves) with at most kSoloTiles

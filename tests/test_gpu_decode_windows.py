@@ -1,39 +1,83 @@
 """Sliding-window decode launches that give a sequence's whole window to one work-group
-(its waves merge in LDS, no merge launch) against the fixed partitions over the same
-inputs, at the edges of the rule that picks them: one sequence, as many as fill the chip,
-windows of one token up to a wave's most tiles, every head size and query group, fp8
-pages, empty contexts, masked pages, and the fused store.
+(its waves merge in LDS, no merge launch), at the edges of the rule that picks them: one
+sequence, as many as fill the chip, windows of one token up to a wave's most tiles, 1, 2, 4
+and 8 shares, every head size and query group, several column blocks per kv head, idle
+waves, fp8 pages, empty contexts, masked pages, and the fused store.  Each case checks which
+launch it gets; a window one tile past the rule takes the balanced schedule.
 
-Both paths sum in fp32 and round P and the row to bf16, so they differ by the rounding of
-P (2^-9 relative each) and of the result: rtol = 2^-7, and atol = 2^-7 of values of N(0, 1)
-rows averaged over the window."""
+Against the fixed partitions over the same inputs and against float64.  All paths sum in
+fp32 and round P and the row to bf16, so two of them differ by the rounding of P (2^-9
+relative each) and of the result: rtol = 2^-7, and atol = 2^-7 of values of N(0, 1) rows
+averaged over the window."""
 from __future__ import annotations
 
 import pytest
 import torch
 
-from fastkernels_amd import ops, workloads
+from fastkernels_amd import _native, ops, workloads
 
 pytestmark = pytest.mark.gpu
 
-# (batch, query heads, kv heads, head size, window_left, fp8)
+# (batch, query heads, kv heads, head size, window_left, fp8, (waves, shares, whole)).  The
+# rule counts (window_left + 16) / 16 + 1 tiles, one more than a window that is a multiple of
+# 16 touches.
 CASES = [
-    (1, 64, 8, 64, 127, False),
-    (1, 32, 8, 128, 0, False),
-    (3, 32, 8, 128, 368, False),    # 24 tiles: the most a few sequences take
-    (5, 16, 2, 256, 176, False),    # 12 tiles, head 256 (at most 4 shares)
-    (40, 64, 8, 64, 128, False),
-    (150, 32, 8, 128, 127, True),   # one share per head
-    (17, 71, 1, 64, 500, False),    # several column blocks per kv head
-    (33, 20, 20, 64, 1136, False),  # 72 tiles over 8 shares
-    (130, 8, 1, 128, 300, True),
-    (2, 40, 1, 256, 15, True),
+    (1, 64, 8, 64, 127, False, (1, 8, True)),
+    (1, 32, 8, 128, 0, False, (1, 8, True)),
+    (3, 32, 8, 128, 367, False, (1, 8, True)),     # 24 tiles: the most a few sequences take
+    (3, 32, 8, 128, 368, False, (8, 1, False)),
+    (5, 16, 2, 256, 175, False, (1, 4, True)),     # 12 tiles, head 256 (at most 4 shares)
+    (5, 16, 2, 256, 176, False, (2, 1, False)),
+    (40, 64, 8, 64, 128, False, (2, 4, True)),
+    (150, 32, 8, 128, 127, True, (8, 1, True)),    # one share per head, 9 tiles
+    (150, 32, 8, 128, 128, False, (4, 2, True)),
+    (17, 71, 1, 64, 367, False, (1, 8, True)),     # five column blocks of one kv head
+    (210, 71, 1, 64, 127, False, (4, 1, True)),    # ... in work-groups of 4: 3 idle waves
+    (103, 71, 1, 64, 271, False, (4, 2, True)),    # 18 tiles over 2 shares, 3 idle heads
+    (52, 71, 1, 64, 559, False, (2, 4, True)),     # 36 tiles over 4 shares, 1 idle head
+    (33, 20, 20, 64, 1135, False, (1, 8, True)),   # 72 tiles over 8 shares
+    (33, 20, 20, 64, 1136, False, (8, 1, False)),
+    (25, 20, 20, 64, 1135, True, (1, 8, True)),    # fp8: 500 work-groups of 8 shares
+    (26, 20, 20, 64, 1135, True, (8, 1, False)),   # 520: past two per CU
+    (260, 16, 2, 256, 300, False, (1, 4, True)),
+    (130, 8, 1, 128, 300, True, (1, 8, True)),
+    (2, 40, 1, 256, 15, True, (1, 4, True)),
 ]
 
 
-@pytest.mark.parametrize("batch,hq,hk,d,window,fp8", CASES)
-def test_whole_windows_match_partitions(cuda, batch, hq, hk, d, window, fp8):
+def _float64(case, bt, lens, window, sinks, fp8):
+    """The rows in float64: keys of the window on readable pages, the sink in the sum."""
+    hk, d = case.k_cache.shape[2:]
+    b, hq = case.q.shape[:2]
+    kc, vc = case.k_cache.float(), case.v_cache.float()
+    if fp8:
+        kc, vc = kc * case.k_scale.view(1, 1, -1, 1), vc * case.v_scale.view(1, 1, -1, 1)
+    kc, vc = kc.view(-1, hk, d).double(), vc.view(-1, hk, d).double()
+    page = case.k_cache.shape[1]
+    out = torch.zeros(b, hq, d, dtype=torch.float64, device=case.q.device)
+    for i, n in enumerate(lens):
+        if n == 0:
+            continue
+        pos = torch.arange(max(0, n - 1 - window), n, device=case.q.device)
+        pg = bt[i].long()[pos // page]
+        slot = (pg * page + pos % page)[pg >= 0]
+        k, v = (t[slot].transpose(0, 1).contiguous() for t in (kc, vc))  # [hk, keys, d]
+        q = case.q[i].double().view(hk, hq // hk, d)
+        s = torch.matmul(q, k.transpose(1, 2).contiguous()) * case.scale
+        s = torch.cat([s, sinks.double().view(hk, hq // hk, 1)], -1)
+        p = torch.softmax(s, -1)[..., :-1].contiguous()
+        out[i] = torch.matmul(p, v).view(hq, d)
+    return out
+
+
+@pytest.mark.parametrize("batch,hq,hk,d,window,fp8,launch", CASES)
+def test_whole_windows_match_partitions(cuda, batch, hq, hk, d, window, fp8, launch):
     print(f"windows {batch} {hq}/{hk}/{d} {window} fp8={fp8}", flush=True)
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the expected launches are those of 256 CUs")
+    plan = _native.plan(batch, hq, hk, d, 1500, 0)
+    assert _native.decode_shape(batch, hq, hk, d, _native.FK_DTYPE_FP8_E4M3FN if fp8 else
+                                _native.FK_DTYPE_BF16, window, plan[0], plan[1]) == launch
     lens = [(977 * i * i + 31 * i) % 1500 for i in range(batch)]  # 0 first, then mixed
     if batch == 1:
         lens = [1203]
@@ -58,6 +102,8 @@ def test_whole_windows_match_partitions(cuda, batch, hq, hk, d, window, fp8):
         outs.append(out.float())
     assert torch.isfinite(outs[0]).all()
     torch.testing.assert_close(outs[0], outs[1], rtol=2 ** -7, atol=2 ** -7)
+    torch.testing.assert_close(outs[0].double(), _float64(case, bt, lens, window, sinks, fp8),
+                               rtol=2 ** -7, atol=2 ** -7)
     for b in range(batch):
         if lens[b] == 0:
             assert not outs[0][b].any()

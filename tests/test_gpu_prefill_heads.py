@@ -230,3 +230,25 @@ def test_flash_attn_prefill_candidate_vision_head_80(cuda):
     torch.cuda.synchronize()
     ref = _oracle_dense(q, k, v, cu, cu, 80 ** -0.5, False)
     _close(out.view(-1, 16, 80), ref, 1e-2, "vision head 80")
+
+
+@pytest.mark.parametrize("d,dv", [(80, 80), (128, 128), (192, 128)])
+def test_varlen_row_strides_near_the_32bit_bound(cuda, d, dv):
+    """Dense rows just under 2^32 / 16 bytes apart (the kernel addresses a tile's 16 rows by
+    32-bit offsets): tiles past 2^31 bytes, a tile that runs past the last row, sequences
+    that start inside one; keys and values are columns of one buffer."""
+    _flush(f"varlen row strides near 2^28 bytes {d}/{dv}")
+    q_lens, k_lens, h = [20, 3, 7], [21, 3, 9], 2
+    stride = ((1 << 28) - 4096) // 2  # elements; 16 rows span 2^32 - 2^16 bytes
+    rows = sum(k_lens)
+    q, k, v, cu_q, cu_k = _dense(cuda, q_lens, k_lens, h, h, d, dv, seed=77 + d)
+    buf = torch.empty((rows - 1) * stride + h * (d + dv), dtype=torch.bfloat16, device=cuda)
+    kw = buf.as_strided((rows, h, d), (stride, d, 1))
+    vw = buf.as_strided((rows, h, dv), (stride, dv, 1), h * d)
+    kw.copy_(k)
+    vw.copy_(v)
+    for causal in (True, False):
+        ref, ref_lse = _oracle_dense(q, k, v, cu_q, cu_k, d ** -0.5, causal, lse=True)
+        out, lse = _run_dense(q, kw, vw, cu_q, cu_k, 20, d ** -0.5, causal, lse=True, max_k=21)
+        _close(out, ref, 1e-2, f"causal={causal}")
+        _lse_close(lse, ref_lse, f"lse causal={causal}")
