@@ -51,12 +51,13 @@ struct PrefillShape {
 // MLA's head sizes (one_col_block_built): two column blocks a wave, or one.  Two serve 32
 // queries with each K / V byte read from LDS but make half as many work-groups; with too
 // few of them CUs stay idle and each one's block takes longer.  Two where their
-// work-groups (a causal pair counts as one) pass 5/8 of the CUs, or their keys are long
+// work-groups (a causal pair counts as one) pass half of the CUs, or their keys are long
 // enough that parts of them make up for it: 2^18 keys over all work-groups, twice that for
 // causal pairs, which see half.  A block of 128 of at most 64 queries would be half empty:
 // one.  Measured on one box, us, one / two (heads of 192 / 128):
 //   causal, 16 heads: 1x256 13.2 / 20.1, 1x1024 27 / 33, 1x2048 43 / 48, 4x512 20 / 27,
-//     32x33 7.3 / 8.8; 1x3000 111 / 75, 4x1024 42.2 / 39.5, 16x400 47 / 40
+//     32x33 7.3 / 8.8; 877 and 1200 47 / 40, 1x3000 111 / 75, 4x1024 42.2 / 39.5, 16x400
+//     47 / 40
 //   not causal, 16 heads: 1x512 over 1024 22 / 26, 1x1024 over 1024 23 / 28; 1x512 over
 //     4096 44 / 39, 1x2000 over 2000 61 / 51, 8x200 over 1000 35 / 32; 128 heads: 4x256
 //     over 512 83 / 67, 8x200 over 1000 300 / 210
@@ -68,7 +69,7 @@ bool two_col_blocks(int64_t batch, int64_t total_q, int64_t max_seqlen_q, int64_
   if (total_q > 0) blocks = std::min(blocks, total_q / wg_tokens + batch);
   const int64_t wgs = grid_x * (pairs ? (blocks + 1) / 2 : blocks);
   const int64_t keys = std::max(max_seqlen_k, max_seqlen_q);
-  return 8 * wgs >= 5LL * num_cus() || wgs * keys >= (int64_t(1) << (pairs ? 19 : 18));
+  return 2 * wgs > num_cus() || wgs * keys >= (int64_t(1) << (pairs ? 19 : 18));
 }
 
 // total_q: the rows of q, or 0 if unknown.
