@@ -62,24 +62,15 @@ __device__ __forceinline__ uint32_t hi_pair(uint32_t a, uint32_t b) {
 }
 
 // 4 OCP e4m3fn bytes -> 4 bf16 of the same values (exact: the scaled conversion
-// with a scale of one, two elements an instruction).
+// with a scale of one, two elements an instruction).  By way of fp32 (four instructions)
+// K at head size 128 is up to 4 % faster where the balanced decode schedule gives a wave
+// few tiles (64 / 8 / 128 heads, us, scaled / fp32: 16 x (1333 .. 4000) 28.6 / 27.6, 4 x
+// (5333 .. 16000) 29.4 / 28.8) and slower where it gives it many (8 x 131072 371.5 /
+// 371.9, run to run 0.1 %; 8 / 1 / 128 heads 4 x (43690 .. 131072) 31.8 / 32.5): not taken.
 __device__ __forceinline__ uint2 fp8x4_to_bf16x4(uint32_t w) {
   return make_uint2(
       __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.f, false)),
       __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.f, true)));
-}
-
-// The same values by way of fp32, four instructions instead of two.  K at head size 128
-// takes it under the balanced decode schedule: 64 / 8 / 128 heads, fp8 pages, us, two ->
-// four instructions: 16 x (1333 .. 4000) 28.4 -> 27.2, 4 x (5333 .. 16000) 29.5 -> 28.7, 16 x
-// (5333 .. 16000) 78.9 -> 79.4; at 64 and 256 four cost 5 to 10 % of the long contexts, and
-// in short whole windows up to 6 %.
-__device__ __forceinline__ uint2 fp8x4_to_bf16x4_by_f32(uint32_t w) {
-  const auto lo = __builtin_amdgcn_cvt_pk_f32_fp8(w, false);
-  const auto hi = __builtin_amdgcn_cvt_pk_f32_fp8(w, true);
-  const bf16x2_t a = {static_cast<__bf16>(lo[0]), static_cast<__bf16>(lo[1])};
-  const bf16x2_t b = {static_cast<__bf16>(hi[0]), static_cast<__bf16>(hi[1])};
-  return make_uint2(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b));
 }
 
 // KV loads (plain cached loads: marking them non-temporal measured slower).
@@ -196,8 +187,8 @@ struct DTile {
 };
 
 // K operand chunks (bf16, dims as described at DTile) of a loaded tile; fp8
-// bytes are converted exactly (fp8x4_to_bf16x4, or with kByF32 through fp32).
-template <bool kByF32, bool kFp8, int D>
+// bytes are converted exactly (fp8x4_to_bf16x4).
+template <bool kFp8, int D>
 __device__ __forceinline__ void k_chunks_d(const DTile<kFp8, D>& t, uint4 (&kc)[D / 32]) {
   if constexpr (!kFp8) {
 #pragma unroll
@@ -209,8 +200,8 @@ __device__ __forceinline__ void k_chunks_d(const DTile<kFp8, D>& t, uint4 (&kc)[
       const uint4& src = t.k[c >> 1];
       const uint32_t w0 = (c & 1) ? src.z : src.x;
       const uint32_t w1 = (c & 1) ? src.w : src.y;
-      const uint2 lo = kByF32 ? fp8x4_to_bf16x4_by_f32(w0) : fp8x4_to_bf16x4(w0);
-      const uint2 hi = kByF32 ? fp8x4_to_bf16x4_by_f32(w1) : fp8x4_to_bf16x4(w1);
+      const uint2 lo = fp8x4_to_bf16x4(w0);
+      const uint2 hi = fp8x4_to_bf16x4(w1);
       kc[c] = make_uint4(lo.x, lo.y, hi.x, hi.y);
     }
   }

@@ -305,8 +305,7 @@ __device__ __forceinline__ uint32_t lane_word(uint32_t v, int src) {
 // and the tile loop that streams a token range [tok_begin, tok_end) of a
 // sequence through it (tok_begin a multiple of 16).  Lane (r, g) of the O
 // accumulators holds O[column 4g + i][dims (D/16) r .. (D/16) r + D/16 - 1].
-// kBalanced: the balanced schedule's (it picks the fp8 conversion of K).
-template <int kG, int D, bool kFp8, int U, bool kStore, bool kBalanced>
+template <int kG, int D, bool kFp8, int U, bool kStore>
 struct WaveState {
   static constexpr int kKc = D / 32;  // K chunks per row (QK^T MFMAs per tile)
   static constexpr int kSl = D / 16;  // P.V slices; also dims per lane
@@ -469,7 +468,7 @@ struct WaveState {
         return;
       }
       uint4 kc[kKc];
-      k_chunks_d<kBalanced && D == 128>(cur, kc);
+      k_chunks_d(cur, kc);
       const floatx4_t acc = qk_scores_n(kc, qb);
       // A tile wholly inside the visible keys on a readable page (every tile but
       // those at a segment's edges) needs no mask: one wave-uniform test skips
@@ -720,7 +719,7 @@ __attribute__((amdgpu_waves_per_eu(FK_DECODE_WAVES_PER_EU))) void paged_decode_p
     // window's first key; one wholly before it streams nothing and leaves an
     // empty partial (max -inf, sum 0).
     const int lo = key_lo(P, ctx);
-    using WS = WaveState<kG, D, kFp8, U, kStore, false>;
+    using WS = WaveState<kG, D, kFp8, U, kStore>;
     WS st;
     const int seg_begin = max(tok_begin, lo & ~(kTile - 1));
     if (P.split == 1) {
@@ -850,7 +849,7 @@ __attribute__((amdgpu_waves_per_eu(FK_DECODE_WAVES_PER_EU))) void paged_decode_b
       const int mid = (lo + hi) >> 1;
       if (toff[mid] <= t_lo) lo = mid; else hi = mid;
     }
-    using WS = WaveState<kG, D, kFp8, U, kStore, true>;
+    using WS = WaveState<kG, D, kFp8, U, kStore>;
     WS st;
     for (int b = lo; b < batch && toff[b] < t_hi; ++b) {
       const int s_lo = max(t_lo, toff[b]) - toff[b];
