@@ -42,10 +42,10 @@ struct PrefillShape {
   int64_t qblocks;    // query blocks per sequence (grid z before the key parts)
   bool may_pair;      // causal pairs of blocks may occur
   int hsplit;         // work-groups per kv head (head groups of up to 4)
-  int ks;           // key parts within a work-group (1 or 2)
-  int xs;           // key parts over work-groups (1: none), with a workspace
-  int ks_plain;     // ks of the same call without a workspace (xs = 1)
-  bool part_f32;    // the key parts' O in fp32 rather than bf16
+  int ks;             // key parts within a work-group (1 or 2)
+  int xs;             // key parts over work-groups (1: none), with a workspace
+  int ks_plain;       // ks of the same call without a workspace (xs = 1)
+  bool part_f32;      // the key parts' O in fp32 rather than bf16
 };
 
 // MLA's head sizes (one_col_block_built): two column blocks a wave, or one.  Two serve 32
@@ -74,8 +74,8 @@ bool two_col_blocks(int64_t batch, int64_t total_q, int64_t max_seqlen_q, int64_
 
 // total_q: the rows of q, or 0 if unknown.
 PrefillShape prefill_shape(bool paged, bool fp8, int64_t batch, int64_t total_q,
-                           int64_t max_seqlen_q, int64_t max_seqlen_k, int num_heads, int num_kv_heads, int head_size,
-                           int head_size_v, int causal) {
+                           int64_t max_seqlen_q, int64_t max_seqlen_k, int num_heads,
+                           int num_kv_heads, int head_size, int head_size_v, int causal) {
   PrefillShape sh;
   const int gqa = num_heads / num_kv_heads;
   const int hw = gqa < kPrefillWaves ? gqa : kPrefillWaves;  // query heads per work-group
@@ -568,8 +568,8 @@ extern "C" int fk_prefill_shape(int paged, int kv_dtype, int64_t batch, int64_t 
              num_kv_heads);
   const bool fp8 = kv_dtype == FK_DTYPE_FP8_E4M3FN;
   fk::PrefillShape sh =
-      fk::prefill_shape(paged != 0, fp8, batch, with_workspace ? total_q : 0, max_seqlen_q, max_seqlen_k, num_heads,
-                        num_kv_heads, head_size, head_size_v, causal);
+      fk::prefill_shape(paged != 0, fp8, batch, with_workspace ? total_q : 0, max_seqlen_q,
+                        max_seqlen_k, num_heads, num_kv_heads, head_size, head_size_v, causal);
   if (!with_workspace) {
     sh.xs = 1;
     sh.ks = sh.ks_plain;

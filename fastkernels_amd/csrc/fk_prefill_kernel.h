@@ -96,7 +96,7 @@ struct PrefillParams {
   int64_t part_rows;  // rows of q (at least cu_seqlens_q[batch])
   int num_heads;
   // Longest items first (0: off, the grid's y is the sequence and z the query
-  // block): the number of sequences, at most 64; the grid's y is then the rank of
+  // block; prefill_order() of the launch decides): the number of sequences, at most 64; the grid's y is then the rank of
   // the item (sequence, query block or pair) in descending order of the
   // sequence's key stages (x P.xs key parts, the part fastest).
   int lpt;
@@ -383,7 +383,8 @@ __device__ __forceinline__ void lds_v_slice2(const uint8_t* buf, int tt, int d, 
 // time share its keys in L2.  Lane b holds sequence b (P.lpt of them, at most
 // 64): its start in the order is the item count of the sequences before it.
 // With the sequences side by side in the grid (block index slowest), the last
-// blocks dispatched were the longest sequences': same box, us, before -> after:
+// blocks dispatched were the longest sequences'.  Where the launch gains by this order
+// (prefill_order() holds the rule and where it loses), same box, us, before -> after:
 // 5 ragged chunks (418 .. 700 over 3191 .. 6000) 384 -> 325, a vision encoder's
 // 1116 .. 3000 tokens (16 heads of 80) 307 -> 224, 13 fp8 prompts of 160 .. 1100
 // 152 -> 139, MLA chunks (2 x 16 heads 192 / 128) 292 -> 249, one prompt unchanged.
@@ -481,10 +482,11 @@ paged_prefill_kernel(PrefillParams P, const int32_t* __restrict__ block_tables,
   constexpr int kStageAll = kKS * kHalfBytes;
   constexpr int kXBytes = kKS > 1 ? kPrefillWaves * kXFloats * 4 : 0;
   __shared__ __align__(16) uint8_t lds_all[kStageAll > kXBytes ? kStageAll : kXBytes];
-  // Grid: x = kv head (x hsplit), y = sequence, z = query block (x P.xs key
-  // parts, the part fastest).  The block index varies slowest, so the
-  // work-groups that have work (low z when blocks are paired) are dispatched
-  // first and spread over every CU.
+  // Grid: x = kv head (x hsplit).  In the grid's own order (P.lpt == 0) y = sequence
+  // and z = query block (x P.xs key parts, the part fastest): the block index varies
+  // slowest, so the work-groups that have work (low z when blocks are paired) are
+  // dispatched first and spread over every CU.  Longest first (P.lpt > 0) y = the
+  // item's rank (x P.xs key parts, the part fastest), z = 1.
   const int hw = P.gqa < kPrefillWaves ? P.gqa : kPrefillWaves;  // heads per work-group
   const int qs = kPrefillWaves / hw;                             // query blocks per work-group
   const int hsplit = (P.gqa + hw - 1) / hw;

@@ -28,7 +28,10 @@ __device__ __forceinline__ float silu_f32(float g) {
 // last-level cache holds (kStreamBytes), where keeping lines only evicts others:
 // same box, us, 8192 x 12288 bf16 (604 MB) 114.5 -> 103 (5.28 -> 5.87 TB/s), 4000 x
 // 12288 (295 MB) 56.2 -> 50, 3000 x 28672 (516 MB) 99 -> 92.  Below it they cost
-// what the cache holds: 1000 x 12288 (74 MB) 12.1 -> 14.
+// what the cache holds: 1000 x 12288 (74 MB) 12.1 -> 14.  The line is where buffers in
+// turn stop fitting: at 280 MB a call whose input another kernel wrote and whose output
+// the next one reads takes 162 -> 156 streamed, one on cold buffers 133 -> 101; only the
+// same buffers over and over, which the cache still mostly holds, lose (46 -> 49).
 constexpr int64_t kStreamBytes = int64_t(256) << 20;
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 template <bool kStream>

@@ -210,7 +210,10 @@ int fk_paged_decode(void* out, int64_t out_row_stride, const void* q, int64_t q_
 /* The two launches fk_paged_decode makes, exposed so a profiler or benchmark can
  * time them separately.  Same arguments as fk_paged_decode.  The partials launch
  * finishes every sequence it holds whole and writes partials for the rest; the
- * reduce launch merges those partials and writes zero rows for empty sequences. */
+ * reduce launch merges those partials and writes zero rows for empty sequences.
+ * Where the partials launch gives every sequence to one work-group whole
+ * (fk_paged_decode_shape's whole windows), it writes all rows, the empty sequences'
+ * zeros too, and the reduce launch does nothing. */
 int fk_paged_decode_partials(void* out, int64_t out_row_stride, const void* q,
                              int64_t q_row_stride, const void* k_cache, const void* v_cache,
                              int kv_dtype, const float* k_scale, const float* v_scale,
@@ -276,8 +279,9 @@ int fk_store_kvcache_convert(const void* key, int64_t key_row_stride, const void
  * query j to keys [k_len - q_len + j - window_left, k_len - q_len + j]; -1 = no window.
  * sinks: NULL or device fp32 [num_heads] attention-sink logits (s_aux), joining each
  * row's softmax denominator as in fk_paged_decode.
- * max_seqlen_q bounds every chunk (it sizes the grid; at most 65535 blocks of 32
- * query tokens, 128 for GQA group 1).  max_seqlen_k (flash_attn_varlen_func's
+ * max_seqlen_q bounds every chunk (it sizes the grid; at most 65535 query blocks, of 32
+ * tokens at GQA group 3 and up, 64 at 2, 128 at 1; half of that at head size 256
+ * and in short MLA launches: fk_prefill_shape's wg_tokens).  max_seqlen_k (flash_attn_varlen_func's
  * max_seqlen_k): a bound on every sequence's key count, or 0 if unknown; it only
  * chooses the launch shape (with few query blocks, each block's keys are split over
  * two halves of a work-group and merged).  num_heads any multiple of num_kv_heads.
@@ -332,8 +336,8 @@ int fk_varlen_prefill(void* out, int64_t out_row_stride, const void* q, int64_t 
  * fk_prefill_split_plan: *workspace_bytes = the workspace fk_paged_prefill_ws /
  * fk_varlen_prefill_ws need for these sizes (paged: 1 for the paged entry point,
  * kv_dtype its cache dtype; total_q = rows of q and out, >= cu_seqlens_q[batch]);
- * 0 when the launch does not split (any workspace, or NULL, then gives the plain
- * launch).  The decision uses these host-side bounds only. */
+ * 0 when the launch does not split (a workspace, whatever its size, then only lets
+ * total_q bound the launch).  The decision uses these host-side bounds only. */
 int fk_prefill_split_plan(int paged, int kv_dtype, int64_t batch, int64_t total_q,
                           int64_t max_seqlen_q, int64_t max_seqlen_k, int num_heads,
                           int num_kv_heads, int head_size, int head_size_v, int causal,
@@ -360,8 +364,8 @@ int fk_prefill_shape(int paged, int kv_dtype, int64_t batch, int64_t total_q,
  * unwritten.  Its contents
  * need no initialisation and are scratch after the call; calls that share a
  * workspace must be ordered (the same stream).  Results match the entry point
- * without _ws to rounding (each part's O is kept in bf16 before the division by its
- * sum, its max and sums in fp32, and merged in fp32). */
+ * without _ws to rounding (each part's O is kept in bf16, in fp32 at head sizes 192 /
+ * 128, before the division by its sum, its max and sums in fp32, and merged in fp32). */
 int fk_paged_prefill_ws(void* out, int64_t out_row_stride, const void* q, int64_t q_row_stride,
                         const void* k_cache, const void* v_cache, int kv_dtype,
                         const float* k_scale, const float* v_scale, const int32_t* block_tables,

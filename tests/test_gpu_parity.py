@@ -528,8 +528,9 @@ def c5_outputs(cuda):
 @pytest.mark.parametrize("seqs", [(0, 1), (2, 3), (4, 5), (6, 7)])
 def test_paged_decode_fp8_c5(c5_outputs, seqs):
     """Every C5 sequence against the oracle (two per test, so each oracle leg stays well
-    inside the per-test timeout), for every schedule.  Kernel and oracle both round
-    float(x) * scale to bf16 before the products (_cast_kv_tile)."""
+    inside the per-test timeout), for every schedule.  The oracle rounds
+    float(x) * scale to bf16 before the products (_cast_kv_tile); the kernel multiplies by
+    the scale after them."""
     case, outs = c5_outputs
     _flush(f"paged_decode C5 fp8: oracle for sequences {seqs}")
     seqs = list(seqs)
