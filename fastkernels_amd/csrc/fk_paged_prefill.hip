@@ -203,16 +203,26 @@ PrefillShape prefill_shape(bool paged, bool fp8, int64_t batch, int64_t total_q,
 //   ragged, many: 64 x (60 .. 600) 198 / 213, at 64 / 8 / 64 206 / 255
 //   equal lengths whose keys pass the caches: 64 x 200 over 1000 399 / 372, at 16 / 2 / 256
 //     507 / 378, 64 x 600 at 16 / 2 / 256 512 / 412
+//   prompts nearly alike: 2 x 2000, rows 92 % of the longest's, 77 / 70, 96 % 76 / 74, 100 %
+//     80 / 82; 4 x 1000, 91 % 46 / 42, 96 % 47 / 46, 100 % 49 / 51; 32 x 600, 91 % 157 / 162
+//   chunks of one length over contexts alike / down to 3/4 / down to 1/4 of the longest:
+//     16 x 256 over 4000 304 / 315, 293 / 288, 266 / 210; 4 x 512 over 4000 147 / 156, 145 /
+//     144, 143 / 139; 32 x 128 over 4000 at 16 / 2 / 256 390 / 390, 406 / 330, 375 / 251; over
+//     shorter ones 16 x 256 over 1000 92 / 102, 88 / 92, 87 / 75, 8 x 512 over 1000 101 /
+//     110, 96 / 103, 91 / 102
 // so it is taken when
 //   - the launch holds more work-groups than CUs (else each has a CU to itself in any
 //     order) of four stages or more, with long keys already at 3/4 of them, and
-//   - the lengths differ: the rows are fewer than 90 % of batch * max_seqlen_q (total_q 0:
-//     unknown, taken as ragged), and the search stays small against an item's stages: at
-//     most 9 stages for each sequence and round of the slots; or
+//   - the lengths differ: the rows are fewer than 90 % of batch * max_seqlen_q, 96 % where
+//     an item's stages are 30 and half of sequences times rounds or more (total_q 0: unknown,
+//     taken as ragged), or 48 stages and more are mostly cached keys, whose lengths the host
+//     does not know (taken as ragged too), and the search stays small against an item's
+//     stages: at most 9 sequences times rounds of the slots for each; or
 //   - over four rounds and more the batch's keys exceed what holds them: the last-level
 //     cache, or, where a work-group computes 64 rows for each key read (head size 256),
 //     the L2s.
-// Head 256 with one or two blocks a sequence in one round keeps its own order (the L2s).
+// Head 256 with one or two blocks a sequence in one round keeps its own order (the L2s)
+// below 96 stages (32 x 32 over 1000 36 / 46; over 1000 .. 4000 99 / 88).
 int prefill_order(const PrefillShape& sh, int xs, int64_t batch, int64_t total_q,
                   int64_t max_seqlen_q, int64_t max_seqlen_k, int num_kv_heads, int head_size,
                   int head_size_v, int window_left, int elem, int64_t items) {
@@ -231,9 +241,14 @@ int prefill_order(const PrefillShape& sh, int xs, int64_t batch, int64_t total_q
   const double key_bytes =
       static_cast<double>(batch) * keys * num_kv_heads * (head_size + head_size_v) * elem;
   if (rounds >= 4 && key_bytes > (few_rows ? 32e6 : 256e6)) return static_cast<int>(batch);
-  if (total_q > 0 && 10 * total_q > 9 * batch * max_seqlen_q) return 0;
-  if (few_rows && num_kv_heads * sh.hsplit % 8 != 0 && rounds <= 1 && sh.qblocks <= 2) return 0;
-  return batch * rounds <= 9 * stages ? static_cast<int>(batch) : 0;
+  const double load = batch * rounds / stages;  // the search against an item's work
+  const bool cached = max_seqlen_k >= 2 * max_seqlen_q && stages >= 48;
+  const int64_t alike = stages >= 30 && load <= 2 ? 96 : 90;  // percent
+  if (!cached && total_q > 0 && 100 * total_q > alike * batch * max_seqlen_q) return 0;
+  if (few_rows && num_kv_heads * sh.hsplit % 8 != 0 && rounds <= 1 && sh.qblocks <= 2 &&
+      stages < 96)
+    return 0;
+  return load <= 9 ? static_cast<int>(batch) : 0;
 }
 
 // Bytes of the work-group key split's partial states (0 without the split).

@@ -188,8 +188,9 @@ def test_decode_work_groups_fit_the_kernel(lib):
 
 def test_prefill_order_rule(lib):
     """fk_prefill_shape's item order: longest first for ragged launches that hold more
-    work-groups than CUs, the grid's own for equal or short lengths, small launches, more
-    than 64 sequences, and where the search would outweigh the items."""
+    work-groups than CUs or chunks over long caches, the grid's own for equal or short
+    lengths, small launches, more than 64 sequences, and where the search would outweigh the
+    items."""
     from fastkernels_amd import _native as N
 
     def order(batch, max_q, total_q, max_k=0, hq=32, hk=8, d=128, causal=True, window=-1, ws=True):
@@ -209,6 +210,12 @@ def test_prefill_order_rule(lib):
     assert order(64, 200, 64 * 200, max_k=300) == 0
     assert order(64, 600, 64 * 600, hq=16, hk=2, d=256) == 64  # head 256: past the L2s
     assert order(16, 1500, 0, ws=False) == 16    # rows unknown: taken as ragged
+    assert order(4, 2000, 7440) == 4             # prompts at 93 % of the longest: long ones
+    assert order(4, 2000, 7840) == 0             # 98 %
+    assert order(32, 300, 8930) == 0             # 93 %, short ones
+    assert order(16, 256, 16 * 256, max_k=4256) == 16  # equal chunks: caches of any lengths
+    assert order(16, 256, 16 * 256, max_k=1256) == 0   # over short ones
+    assert order(16, 256, 16 * 256, max_k=4256, window=500) == 0
 
 
 def test_argument_errors_return_before_launch(lib):
