@@ -52,13 +52,14 @@ struct PrefillShape {
 // queries with each K / V byte read from LDS but make half as many work-groups; with too
 // few of them CUs stay idle and each one's block takes longer.  Two where their
 // work-groups (a causal pair counts as one) pass half of the CUs, or their keys are long
-// enough that parts of them make up for it: 2^18 keys over all work-groups, twice that for
-// causal pairs, which see half.  A block of 128 of at most 64 queries would be half empty:
-// one.  Measured on one box, us, one / two (heads of 192 / 128):
+// enough that parts of them make up for it: 1800 and 2^17 over all work-groups, 2^19 for
+// causal pairs, which see half and run in one part.  A block of 128 of at most 64 queries
+// would be half empty: one.  Measured on one box, us, one / two (heads of 192 / 128):
 //   causal, 16 heads: 1x256 13.2 / 20.1, 1x1024 27 / 33, 1x2048 43 / 48, 4x512 20 / 27,
 //     32x33 7.3 / 8.8; 877 and 1200 47 / 40, 1x3000 111 / 75, 4x1024 42.2 / 39.5, 16x400
 //     47 / 40
-//   not causal, 16 heads: 1x512 over 1024 22 / 26, 1x1024 over 1024 23 / 28; 1x512 over
+//   not causal, 16 heads: 1x512 over 1024 22 / 26, 1x1024 over 1024 23 / 28, 92 and 95 over
+//     745 17 / 19; 598 over 2279 43 / 34, 62 .. 107 over 3340 37 / 27; 1x512 over
 //     4096 44 / 39, 1x2000 over 2000 61 / 51, 8x200 over 1000 35 / 32; 128 heads: 4x256
 //     over 512 83 / 67, 8x200 over 1000 300 / 210
 bool two_col_blocks(int64_t batch, int64_t total_q, int64_t max_seqlen_q, int64_t max_seqlen_k,
@@ -69,7 +70,8 @@ bool two_col_blocks(int64_t batch, int64_t total_q, int64_t max_seqlen_q, int64_
   if (total_q > 0) blocks = std::min(blocks, total_q / wg_tokens + batch);
   const int64_t wgs = grid_x * (pairs ? (blocks + 1) / 2 : blocks);
   const int64_t keys = std::max(max_seqlen_k, max_seqlen_q);
-  return 2 * wgs > num_cus() || wgs * keys >= (int64_t(1) << (pairs ? 19 : 18));
+  return 2 * wgs > num_cus() ||
+         (pairs ? wgs * keys >= int64_t(1) << 19 : keys >= 1800 && wgs * keys >= int64_t(1) << 17);
 }
 
 // total_q: the rows of q, or 0 if unknown.
@@ -210,22 +212,28 @@ PrefillShape prefill_shape(bool paged, bool fp8, int64_t batch, int64_t total_q,
 //     144, 143 / 139; 32 x 128 over 4000 at 16 / 2 / 256 390 / 390, 406 / 330, 375 / 251; over
 //     shorter ones 16 x 256 over 1000 92 / 102, 88 / 92, 87 / 75, 8 x 512 over 1000 101 /
 //     110, 96 / 103, 91 / 102
+//   not causal, 16 heads of 72, lengths alike: 16 x 1500 307 / 238, 32 x 700 167 / 131, 64 x
+//     300 93 / 86, 8 x 1500 (61 MB) 122 / 123, 16 x 300 22 / 22, 32 x 150 21 / 25; 20 heads of
+//     64 16 x 1500 238 / 244; 16 heads of 192 / 128 over other keys: 1226 and 1217 over 1454 and
+//     2192 99 / 76, 4 x 1200 over 950 .. 1600 114 / 92, 3 x 1070 .. 1250 over 180 .. 275 30 / 30
 // so it is taken when
 //   - the launch holds more work-groups than CUs (else each has a CU to itself in any
 //     order) of four stages or more, with long keys already at 3/4 of them, and
 //   - the lengths differ: the rows are fewer than 90 % of batch * max_seqlen_q, 96 % where
 //     an item's stages are 30 and half of sequences times rounds or more (total_q 0: unknown,
-//     taken as ragged), or 48 stages and more are mostly cached keys, whose lengths the host
-//     does not know (taken as ragged too), and the search stays small against an item's
-//     stages: at most 9 sequences times rounds of the slots for each; or
+//     taken as ragged), or 48 stages and more are mostly cached keys, or, not causal, 16 and
+//     more are of other lengths than the queries: the host does not know the keys' lengths
+//     (taken as ragged too).  And the search stays small against an item's stages: at most
+//     9 sequences times rounds of the slots for each; or
 //   - over four rounds and more the batch's keys exceed what holds them: the last-level
 //     cache, or, where a work-group computes 64 rows for each key read (head size 256),
-//     the L2s.
+//     the L2s; not causal (no light last blocks to lose) from three rounds, 8 stages and
+//     48 MB on where a head's blocks stay on one XCD.
 // Head 256 with one or two blocks a sequence in one round keeps its own order (the L2s)
 // below 96 stages (32 x 32 over 1000 36 / 46; over 1000 .. 4000 99 / 88).
 int prefill_order(const PrefillShape& sh, int xs, int64_t batch, int64_t total_q,
                   int64_t max_seqlen_q, int64_t max_seqlen_k, int num_kv_heads, int head_size,
-                  int head_size_v, int window_left, int elem, int64_t items) {
+                  int head_size_v, int causal, int window_left, int elem, int64_t items) {
   if (batch > 64 || items * xs > 65535) return 0;
   if (batch == 1) return 1;  // (its blocks in order, at no cost)
   const double ncu = num_cus();
@@ -242,7 +250,12 @@ int prefill_order(const PrefillShape& sh, int xs, int64_t batch, int64_t total_q
       static_cast<double>(batch) * keys * num_kv_heads * (head_size + head_size_v) * elem;
   if (rounds >= 4 && key_bytes > (few_rows ? 32e6 : 256e6)) return static_cast<int>(batch);
   const double load = batch * rounds / stages;  // the search against an item's work
-  const bool cached = max_seqlen_k >= 2 * max_seqlen_q && stages >= 48;
+  if (!causal && num_kv_heads * sh.hsplit % 8 == 0 && rounds >= 3 && stages >= 8 &&
+      key_bytes > 48e6)
+    return static_cast<int>(batch);
+  // Keys whose lengths the bounds do not tell.
+  const bool cached = causal ? max_seqlen_k >= 2 * max_seqlen_q && stages >= 48
+                             : max_seqlen_k > 0 && max_seqlen_k != max_seqlen_q && stages >= 16;
   const int64_t alike = stages >= 30 && load <= 2 ? 96 : 90;  // percent
   if (!cached && total_q > 0 && 100 * total_q > alike * batch * max_seqlen_q) return 0;
   if (few_rows && num_kv_heads * sh.hsplit % 8 != 0 && rounds <= 1 && sh.qblocks <= 2 &&
@@ -466,7 +479,7 @@ int prefill_entry(const char* name, bool paged, void* out, int64_t out_row_strid
   if (workspace != nullptr && total_q > 0)
     items = std::min(items, total_q / sh.wg_tokens + batch);
   P.lpt = prefill_order(sh, sh.xs, batch, workspace ? total_q : 0, max_seqlen_q, max_seqlen_k,
-                        num_kv_heads, head_size, head_size_v, window_left,
+                        num_kv_heads, head_size, head_size_v, causal, window_left,
                         static_cast<int>(elem), items);
   const dim3 grid =
       P.lpt ? dim3(static_cast<unsigned>(num_kv_heads * sh.hsplit),
@@ -597,7 +610,7 @@ extern "C" int fk_prefill_shape(int paged, int kv_dtype, int64_t batch, int64_t 
   *parts = sh.xs;
   *longest_first =
       fk::prefill_order(sh, sh.xs, batch, total_q, max_seqlen_q, max_seqlen_k, num_kv_heads,
-                        head_size, head_size_v, window_left, fp8 ? 1 : 2, items);
+                        head_size, head_size_v, causal, window_left, fp8 ? 1 : 2, items);
   return FK_OK;
 }
 

@@ -216,6 +216,13 @@ def test_prefill_order_rule(lib):
     assert order(16, 256, 16 * 256, max_k=4256) == 16  # equal chunks: caches of any lengths
     assert order(16, 256, 16 * 256, max_k=1256) == 0   # over short ones
     assert order(16, 256, 16 * 256, max_k=4256, window=500) == 0
+    # Not causal: keys of other lengths than the queries, and keys past the L2s whose heads
+    # stay on one XCD each.
+    assert order(4, 1200, 4800, max_k=1600, hq=16, hk=16, causal=False) == 4
+    assert order(4, 1200, 4800, hq=16, hk=16, causal=False) == 0
+    assert order(32, 700, 32 * 700, hq=16, hk=16, d=64, causal=False) == 32
+    assert order(32, 700, 32 * 700, hq=20, hk=20, d=64, causal=False) == 0
+    assert order(64, 150, 64 * 150, hq=16, hk=16, d=128, causal=False) == 0  # short
 
 
 def test_argument_errors_return_before_launch(lib):
