@@ -491,23 +491,19 @@ PREFILL_SPLIT = True
 
 
 def _split_workspace(q, paged, kv_dtype, batch, max_seqlen_q, max_seqlen_k, hk, dv, causal):
-    """The workspace of the prefill's work-group key split (fk_prefill_split_plan), from
-    torch's allocator on q's stream, or None when the launch does not split."""
+    """(workspace, bytes) of the _ws entry points: the prefill's work-group key split
+    (fk_prefill_split_plan), from torch's allocator on q's stream.  A launch that does not
+    split takes any workspace of 0 bytes, which it never reads or writes; one that is not
+    NULL (q here) lets q's row count bound the grid (64 prompts of 16 .. 2000 tokens:
+    1115 -> 1025 us)."""
     if not PREFILL_SPLIT:
-        return None
+        return None, 0
     nbytes = _native.prefill_split_bytes(paged, kv_dtype, batch, q.shape[0], int(max_seqlen_q),
                                          int(max_seqlen_k), q.shape[1], hk, q.shape[2], dv,
                                          causal)
-    return torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes > 0 else None
-
-
-def _workspace_args(ws, q):
-    """(workspace, bytes) of the _ws entry points.  A launch that does not split takes any
-    workspace of 0 bytes; one that is not NULL lets q's row count bound the grid (64
-    prompts of 16 .. 2000 tokens: 1115 -> 1025 us)."""
-    if ws is not None:
-        return ws.data_ptr(), ws.numel()
-    return (q.data_ptr() if PREFILL_SPLIT else None), 0
+    if nbytes > 0:
+        return torch.empty(nbytes, dtype=torch.uint8, device=q.device), nbytes
+    return q, 0
 
 
 def paged_prefill(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor,
@@ -552,14 +548,15 @@ def paged_prefill(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor,
         return
     nb, bs = k_cache.shape[:2]
     kv_dtype = _native.FK_DTYPE_FP8_E4M3FN if k_cache.dtype == _FP8 else _native.FK_DTYPE_BF16
-    ws = _split_workspace(q, True, kv_dtype, batch, max_seqlen_q, max_seqlen_k, hk, dv, causal)
+    ws, ws_bytes = _split_workspace(q, True, kv_dtype, batch, max_seqlen_q, max_seqlen_k, hk,
+                                    dv, causal)
     _native.call("fk_paged_prefill_ws", _ptr(out), out.stride(0), _ptr(q), q.stride(0),
                  _ptr(k_cache), _ptr(v_cache), kv_dtype,
                  _ptr(k_scale), _ptr(v_scale), _ptr(block_table), block_table.stride(0),
                  _ptr(cu_seqlens_q), _ptr(cu_seqlens_k), batch, int(max_seqlen_q),
                  int(max_seqlen_k), q.shape[1], hk, q.shape[2], dv, bs, nb,
                  float(softmax_scale), int(bool(causal)), int(window_left), _ptr(sinks),
-                 q.shape[0], *_workspace_args(ws, q), _stream(q))
+                 q.shape[0], _ptr(ws), ws_bytes, _stream(q))
 
 
 def varlen_prefill(out: torch.Tensor, q: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
@@ -592,14 +589,14 @@ def varlen_prefill(out: torch.Tensor, q: torch.Tensor, key: torch.Tensor, value:
     batch = cu_seqlens_q.numel() - 1
     if batch <= 0 or q.shape[0] == 0:
         return
-    ws = _split_workspace(q, False, _native.FK_DTYPE_BF16, batch, max_seqlen_q, max_seqlen_k,
-                          key.shape[1], dv, causal)
+    ws, ws_bytes = _split_workspace(q, False, _native.FK_DTYPE_BF16, batch, max_seqlen_q,
+                                    max_seqlen_k, key.shape[1], dv, causal)
     _native.call("fk_varlen_prefill_ws", _ptr(out), out.stride(0), _ptr(q), q.stride(0),
                  _ptr(key), key.stride(0), _ptr(value), value.stride(0), _ptr(cu_seqlens_q),
                  _ptr(cu_seqlens_k), batch, int(max_seqlen_q), int(max_seqlen_k), q.shape[1],
                  key.shape[1], q.shape[2], dv, float(softmax_scale), int(bool(causal)),
                  int(window_left), _ptr(sinks), _ptr(lse), 0 if lse is None else lse.stride(0),
-                 q.shape[0], *_workspace_args(ws, q), _stream(q))
+                 q.shape[0], _ptr(ws), ws_bytes, _stream(q))
 
 
 def paged_decode_phases(out, q, k_cache, v_cache, block_table, cache_seqlens, softmax_scale,
